@@ -79,15 +79,7 @@ constexpr int kMaxRaw = 1024;
 constexpr int kMaxDist = 1024;
 constexpr int kMaxRows = 1024;
 // Stored precision of the fill's output (fem2d_precision): the value types of
-// A and B and the streaming fill's launch shape. The wavefronts of a block
-// share one LDS copy of the Gram library (up to kLibLds values) beside their
-// staged source records. FP64 output: 16 wavefronts and up to 96 KB of
-// library (orders to 8 over three levels of refinement), one block per CU,
-// measured faster than three 8-wavefront blocks with a 32 KB library; FP32
-// output (12 B per entry, more latency-bound) keeps the three smaller blocks
-// per CU. kChunk: CSR entries per work item (256 for all; 512 made the FP32
-// fill faster on Domains of large row groups and slower on Domains of small
-// ones, and the FP64 fill slower on all that were measured).
+// A and B.
 constexpr int kPrecisions = 3;
 template <int kPrecision>
 struct Store;
@@ -96,40 +88,30 @@ struct Store<FEM2D_PRECISION_FP64> {
   using A = double;
   using B = double;
   static constexpr bool kRes = false;  // 16-bit residuals stored beside the values (FP32R)
-  static constexpr int kBlock = 1024;
-  static constexpr int kLibLds = 12288;
-  static constexpr int kChunk = 256;
 };
 template <>
 struct Store<FEM2D_PRECISION_FP32> {
   using A = float;
   using B = float;
   static constexpr bool kRes = false;
-  static constexpr int kBlock = 512;
-  static constexpr int kLibLds = 4096;
-  static constexpr int kChunk = 256;
 };
 template <>
-struct Store<FEM2D_PRECISION_FP32R> {  // 16 B per entry: the FP64 shape
+struct Store<FEM2D_PRECISION_FP32R> {
   using A = float;
   using B = float;
   static constexpr bool kRes = true;
-  static constexpr int kBlock = 1024;
-  static constexpr int kLibLds = 12288;
-  static constexpr int kChunk = 256;
 };
-// Launch shape of the streaming fill: the precision's own (kSmall 0), or 512
-// threads a block with a 4096-value library copy (kSmall 1), which lets three
-// blocks share a CU when the Domain's library is that small
-template <int P, int kSmall>
-struct FillShape {
-  static constexpr int kBlock = kSmall ? 512 : Store<P>::kBlock;
-  static constexpr int kLibLds = kSmall ? 4096 : Store<P>::kLibLds;
-};
-// placements of the fill's Gram library: global memory, an LDS copy in the
-// precision's shape, an LDS copy in the small shape
-enum FillPlace { kPlaceGlobal = 0, kPlaceLds = 1, kPlaceLdsSmall = 2 };
-constexpr int kFillWavesPerSimd = 6;
+// Launch shape of the streaming fill: one block a CU, whose 16 wavefronts share
+// one LDS copy of the Gram library of up to 96 KB (orders to 8 over three levels
+// of refinement) beside 3.6 KB of their own each. Two 8-wavefront blocks with a
+// 32 KB copy each measured the same (93 and 93 us FP64 on 25.7 M entries, 154 and
+// 152 us on 37.6 M in small groups).
+constexpr int kFillBlock = 1024;
+constexpr int kFillLibLds = 12288;
+constexpr int kFillChunk = 512;  // CSR entries per work item, before any tuning
+// placements of the fill's Gram library: global memory, or an LDS copy
+enum FillPlace { kPlaceGlobal = 0, kPlaceLds = 1 };
+constexpr int kFillWavesPerSimd = 4;
 // latency-bound kernels: at most 64 VGPRs, so that 8 wavefronts per SIMD are resident
 constexpr int kLatencyWavesPerSimd = 8;
 constexpr int kMaxDepth = 24;      // h-refinement depth below a base Elem
@@ -210,6 +192,7 @@ struct Work {
   int64_t* row_len;  // [N+1]
   int64_t* row_ptr;  // [N+1]
   double* lib;
+  int lib_tab;           // library values per kind and range: p1 * p1
   int lib_range_stride;  // library values per range: p1 * p1 * kKinds
   int lib_nr;            // ranges of the x axis (the y axis's start at lib_nr)
   const long long* ranges;  // [nr_u + nr_v] sorted keys depth << 32 | index of the sub-ranges, per axis
@@ -221,22 +204,24 @@ struct Work {
   int range_map_v;
   int* err;
   int* n_large;       // row groups handled by the block path
+  int* ticket;        // chunk rounds that the streaming fill's blocks have taken
   int* large_list;
   unsigned char* is_large;
   // per row group, fixed-stride records written by the describe kernel and
   // streamed by the fill kernel (groups of the block path have T = -1)
   int4* meta_hdr;      // [G] T (first row's length), rows, sources, first row
-  double* meta_coef;   // [G * kWS * kCoef] per source: CurlCurl (4) and L2Inner (2) prefactors, then
-                       // int4 {x range base, y range base, k | rel << 1, 0} of the library
-  uint4* meta_col;     // [G * kWC] per candidate column t: column, packed spec of the first and second
-                       // contribution (~0 if none), their sources (bits 0-7 and 8-15)
+  double* meta_coef;   // [G * kWS * kCoef] per source and column direction: the CurlCurl prefactors by row
+                       // direction (2), the L2Inner prefactor and two ints, the byte offsets of the
+                       // source's range on the x and y axes of the library (the y one plus one table)
+  uint4* meta_col;     // [G * kWC] per candidate column t: column, first and second contribution (col_contrib,
+                       // ~0 if none), their library offsets on the y axis (bits 0-15 and 16-31)
   uint2* meta_row;     // [N] per DoF: packed specs on its row group's first / second Elem (written
                        // by the DoF-group scan; a group's rows start at its header's w)
   int meta_cap;        // row groups the records have room for
   int64_t* seg_start;  // [G+1] first CSR entry of each row group
-  int* chunk_first;    // [chunk_cap] row group holding the first entry of each chunk
+  int* chunk_first;    // [chunk_cap] row holding the first entry of each chunk
   long long chunk_cap;
-  int chunk;           // CSR entries per chunk (the stored precision's Store::kChunk)
+  int chunk;           // CSR entries per chunk
   long long n_dofs;
 };
 
@@ -475,10 +460,6 @@ __device__ __forceinline__ T ld_const(const T* base, long long idx) {
   using ConstT = const __attribute__((address_space(4))) T;
   return ((ConstT*)base)[idx];  // only a C-style cast converts to the constant address space
 }
-__device__ __forceinline__ int4 ld_const(const int4* base, long long idx) {
-  const int* p = reinterpret_cast<const int*>(base + idx);
-  return make_int4(ld_const(p, 0), ld_const(p, 1), ld_const(p, 2), ld_const(p, 3));
-}
 
 template <class T>
 __device__ __forceinline__ T ld32(const T* __restrict__ base, unsigned idx) {
@@ -517,6 +498,7 @@ __device__ __forceinline__ void init_body(const Work& w, int n_elems, long long 
   if (t == 0) {
     *w.err = 0;
     *w.n_large = 0;
+    *w.ticket = 0;
   }
 }
 
@@ -870,13 +852,43 @@ struct NestedScan {
   __device__ void store(long long e, long long excl, long long) const { w.nested_ptr[e] = int(excl); }
 };
 
+// Entry p of a row group's segment: row q = max{q : off(q) <= p} with
+// off(q) = q T - q (q - 1) / 2, candidate column t = q + p - off(q). The float
+// root (all operands below 2^24, hardware square root) lands within one row of
+// q; one branch-free step each way fixes it, and the clamp keeps q inside the
+// group's row records whatever the rounding. Returns q and oq = off(q).
+__device__ __forceinline__ void segment_row(int p, int T, int nrows, float bq, int& q, int& oq) {
+  q = int((bq - __builtin_amdgcn_sqrtf(fmaxf(bq * bq - 8.0f * float(p), 0.0f))) * 0.5f);
+  q = min(max(q, 0), nrows - 1);
+  // off(q) = q (2T - q + 1) / 2; both factors stay below 2^24
+  oq = int(__umul24(unsigned(q), unsigned(2 * T - q + 1)) >> 1);
+  const bool down = oq > p && q > 0;
+  q -= down ? 1 : 0;
+  oq -= down ? T - q : 0;
+  const bool up = q + 1 < nrows && oq + (T - q) <= p;
+  oq += up ? T - q : 0;
+  q += up ? 1 : 0;
+}
+
+// First column record and first source record of row group g inside its slots of
+// kWC and kWS records. The slots are multiples of the memory channels' interleaving
+// apart and most groups fill a small part of them: with every group's records at
+// its slots' starts they lay on a few of the channels (and of the memory-side
+// cache's slices), so neighbouring groups start at different multiples of 256 B.
+__device__ __forceinline__ int col_slot(int g, int T) {
+  return ((((g >> 3) & 15) * (((kWC - T) >> 4) + 1)) >> 4) << 4;
+}
+__device__ __forceinline__ int src_slot(int g, int n_src) {
+  return ((((g >> 4) & 7) * (((kWS - n_src) >> 2) + 1)) >> 3) << 2;
+}
+
 // CSR layout by row groups. Item g is the length of group g's segment: row q
 // of a streaming-fill group holds T - q entries, so the segment is
 // nrows T - nrows (nrows - 1) / 2 long; a block-path group sums the row
 // lengths its count kernel wrote. The exclusive sum is the segment's first
-// entry. The store writes the group id for the chunks of w.chunk entries that
-// start inside the segment and, for a block-path group, row_ptr of its rows
-// (the streaming fill writes those of the other groups). The item past the
+// entry. The store writes the row of the first entry of each chunk of w.chunk
+// entries that starts inside the segment and, for a block-path group, row_ptr of
+// its rows (the streaming fill writes those of the other groups). The item past the
 // last group carries nnz and writes the call's status block (nnz, error bits,
 // block-path groups, row groups).
 struct GroupScan {
@@ -907,16 +919,23 @@ struct GroupScan {
     }
     if (*w.err || g >= n_groups) return;  // an invalid view: the group records are not trustworthy
     const int4 hdr = w.meta_hdr[g];
+    const long long C = w.chunk;
+    long long c = (excl + C - 1) / C;
     if (hdr.x <= 0) {  // a block-path group (the streaming fill writes the row pointers of the others)
       const int r0 = w.g_start[g], nrows = w.g_start[g + 1] - r0;
       long long at = excl;
       for (int q = 0; q < nrows; ++q) {
         w.row_ptr[r0 + q] = at;
         at += w.row_len[r0 + q];
+        for (; c * C < at && c < w.chunk_cap; ++c) w.chunk_first[c] = r0 + q;
       }
+      return;
     }
-    const long long C = w.chunk;
-    for (long long c = (excl + C - 1) / C; c * C < excl + len && c < w.chunk_cap; ++c) w.chunk_first[c] = int(g);
+    for (; c * C < excl + len && c < w.chunk_cap; ++c) {
+      int q, oq;
+      segment_row(int(c * C - excl), hdr.x, hdr.y, 2.0f * float(hdr.x) + 1.0f, q, oq);
+      w.chunk_first[c] = hdr.w + q;
+    }
   }
 };
 
@@ -1247,19 +1266,19 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
       int ru, rv;
       double cA[4], cB[2];
       block_coefs(w, P, Q, rel == kLocal, cA, cB, ru, rv);
-      double* out = coef + lane * kCoef;
+      // per column direction: the CurlCurl prefactors by row direction (the p
+      // side of the pair is the column's where the source is an ancestor), the
+      // L2Inner prefactor and the library bases
+      double* out = coef + (src_slot(g, n_src) + lane) * kCoef;
       out[0] = cA[0];
-      out[1] = cA[1];
-      out[2] = cA[2];
-      out[3] = cA[3];
-      out[4] = cB[0];
-      out[5] = cB[1];
-      // library range bases of the pair and which of the group's Elems it uses
-      int* tail = reinterpret_cast<int*>(out + 6);
-      tail[0] = ru * w.lib_range_stride;
-      tail[1] = (w.lib_nr + rv) * w.lib_range_stride;
-      tail[2] = k | (rel << 1);
-      tail[3] = 0;
+      out[1] = rel == kAnc ? cA[1] : cA[2];
+      out[4] = rel == kAnc ? cA[2] : cA[1];
+      out[5] = cA[3];
+      const int2 base = make_int2(8 * (ru * w.lib_range_stride), 8 * ((w.lib_nr + rv) * w.lib_range_stride + w.lib_tab));
+      for (int d = 0; d < 2; ++d) {
+        out[4 * d + 2] = cB[d];
+        *reinterpret_cast<int2*>(out + 4 * d + 3) = base;
+      }
       S.src_info[lane] = k | (rel << 1) | (ru << 3) | (rv << 17);
     }
   }
@@ -1345,6 +1364,42 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
   return 0;
 }
 
+// Where a stored entry finds its two library values. With p the spec on the
+// larger Elem of a nested pair (the ancestor, or the Elem itself) and q the
+// other, pair = 2 dir_p + dir_q, and tab = p1 * p1 values per kind, they are at
+//   x: base_x + i_p p1 + i_q + pair tab,  y: base_y + j_p p1 + j_q + (3 - pair) tab
+// Each sum splits into a part of the source (its range), a part of the column
+// (its order, and its direction's share of pair) and a part of the row, all in
+// bytes, so that the fill adds three words per axis. A column's
+// contribution is one word: whether the source is an ancestor and which of the
+// group's Elems the row's spec is on (bits 3 and 4, the row's variant), its
+// direction (bit 5), the source (bits 6-10) and the x part (bits 16-31); the y part,
+// biased by 2 tab so that it is not negative, comes back in y (the source's y
+// base holds the remaining tab).
+__device__ __forceinline__ unsigned col_contrib(int source, int info, unsigned spec, int tab, unsigned& y) {
+  const bool anc = ((info >> 1) & 3) == kAnc;
+  const unsigned d = spec_dir(spec), dt = d * unsigned(tab);
+  const unsigned x = anc ? spec_ip1(spec) + 2u * dt : spec_i(spec) + dt;
+  y = 8u * (2u * unsigned(tab) + (anc ? spec_jp1(spec) - 2u * dt : spec_j(spec) - dt));
+  return (anc ? 1u << 3 : 0u) | ((unsigned(info) & 1u) << 4) | (d << 5) | (unsigned(source) << 6) | ((8u * x) << 16);
+}
+
+// A row's part of the same sums, for one of its specs, where the row is the q
+// side (the source is an ancestor of the row's Elem) or the p side: x and y in
+// the halves of .x; .y has the direction in bit 0 and the offsets (bytes, x in
+// the low half, y in the high one) from the entry's values to L2Inner's: of two
+// specs of one direction, the table after the one on the axis of their T
+// functions is TT.
+__device__ __forceinline__ uint2 row_variant(unsigned spec, bool anc, int tab) {
+  const int d = int(spec_dir(spec)), dt = d * tab;
+  const int x = anc ? int(spec_i(spec)) + dt : int(spec_ip1(spec)) + 2 * dt;
+  const int y = anc ? int(spec_j(spec)) - dt : int(spec_jp1(spec)) - 2 * dt;
+  return make_uint2((unsigned(8 * x) & 0xffffu) | (unsigned(8 * y) << 16),
+                    d ? unsigned(8 * tab) | 1u : unsigned(8 * tab) << 16);
+}
+static_assert(8 * (kMaxOrder * (kMaxOrder + 1) + 2 * (kMaxOrder + 1) * (kMaxOrder + 1)) < (1 << 15) && kWS <= 32,
+              "library offsets and sources of the fill's records");
+
 // One wavefront per row group: build the candidate set, then write the row
 // lengths and the group's fixed-stride records for the streaming fill:
 // source prefactors and infos, the packed specs of its rows, and for each
@@ -1393,10 +1448,14 @@ __global__ void __launch_bounds__(kBlock, kLatencyWavesPerSimd) k_describe_wave(
         const int m0 = S.dmeta0[a], m1 = S.dmeta1[a];
         uint4 rec;
         rec.x = unsigned(S.dstart[a] + within);
-        rec.y = w.bs_pack[S.src_bs[m0 & 0xff] + (m0 >> 8) + within];
-        rec.z = m1 < 0 ? ~0u : w.bs_pack[S.src_bs[m1 & 0xff] + (m1 >> 8) + within];
-        rec.w = unsigned(m0 & 0xff) | (m1 < 0 ? 0u : unsigned(m1 & 0xff) << 8);
-        w.meta_col[(long long)g * kWC + t] = rec;
+        const int s0 = m0 & 0xff, s1 = m1 & 0xff;
+        unsigned y0, y1 = 0u;
+        rec.y = col_contrib(s0, S.src_info[s0], w.bs_pack[S.src_bs[s0] + (m0 >> 8) + within], w.lib_tab, y0);
+        rec.z = ~0u;
+        if (m1 >= 0)
+          rec.z = col_contrib(s1, S.src_info[s1], w.bs_pack[S.src_bs[s1] + (m1 >> 8) + within], w.lib_tab, y1);
+        rec.w = y0 | (y1 << 16);
+        w.meta_col[(long long)g * kWC + col_slot(g, T) + t] = rec;
       }
     }
     wave_sync();
@@ -1429,109 +1488,6 @@ __device__ __forceinline__ void write_entry(const FillOut& o, long long pos, int
   }
 }
 
-// contribution of one (row spec, column spec) pair through source s of the
-// group; the source record (staged in LDS) holds the prefactors, the library
-// range bases and which of the group's Elems (k) and which relation (rel) the
-// pair has. lib is the Gram library in global memory or its copy in LDS.
-__device__ __forceinline__ void flat_contrib(const double* __restrict__ lib, unsigned tab,
-                                             const double* __restrict__ coef_g, unsigned s, unsigned cbs, uint2 rp,
-                                             double& cc, double& l2) {
-  const unsigned ci = s * unsigned(kCoef);
-  const int4 tail = reinterpret_cast<const int4*>(coef_g)[ci / 2u + 3u];
-  const unsigned rpk = (tail.z & 1) ? rp.y : rp.x;
-  const bool anc = (tail.z >> 1) == kAnc;
-  // the p side of the reference's pair is the ancestor's spec (selected as
-  // whole spec words, so that the field extraction below is branch-free)
-  const unsigned ps = anc ? cbs : rpk, qs = anc ? rpk : cbs;
-  const unsigned pd = spec_dir(ps), qd = spec_dir(qs);
-  const unsigned pair = 2u * pd + qd;
-  // table row a = p's order, entry b = q's order
-  const unsigned ix = unsigned(tail.x) + spec_ip1(ps) + spec_i(qs);
-  const unsigned iy = unsigned(tail.y) + spec_jp1(ps) + spec_j(qs);
-  const double fx = ld32(lib, ix + __umul24(pair, tab));
-  const double fy = ld32(lib, iy + __umul24(3u - pair, tab));
-  cc = coef_g[ci + pair] * fx * fy;
-  // L2Inner (UU, VV only): the TT factor replaces the N N factor's partner on
-  // the axis where the pair has its T functions; read unconditionally
-  const double ftt = ld32(lib, (pd ? ix : iy) + __umul24(unsigned(kTT), tab));
-  const double l2v = (coef_g[ci + 4u + pd] * (pd ? ftt : fx)) * (pd ? fy : ftt);
-  l2 = pd == qd ? l2v : 0.0;
-}
-
-// Entry p of a row group's segment: row q = max{q : off(q) <= p} with
-// off(q) = q T - q (q - 1) / 2, candidate column t = q + p - off(q). The float
-// root (all operands below 2^24, hardware square root) lands within one row of
-// q; one branch-free step each way fixes it, and the clamp keeps q inside the
-// group's row records whatever the rounding. Returns q and oq = off(q).
-__device__ __forceinline__ void segment_row(int p, int T, int nrows, float bq, int& q, int& oq) {
-  q = int((bq - __builtin_amdgcn_sqrtf(fmaxf(bq * bq - 8.0f * float(p), 0.0f))) * 0.5f);
-  q = min(max(q, 0), nrows - 1);
-  // off(q) = q (2T - q + 1) / 2; both factors stay below 2^24
-  oq = int(__umul24(unsigned(q), unsigned(2 * T - q + 1)) >> 1);
-  const bool down = oq > p && q > 0;
-  q -= down ? 1 : 0;
-  oq -= down ? T - q : 0;
-  const bool up = q + 1 < nrows && oq + (T - q) <= p;
-  oq += up ? T - q : 0;
-  q += up ? 1 : 0;
-}
-
-// Moves (q, oq) forward to the row of a later entry p (row q has T - q
-// entries; q stays below nrows, so the loop ends).
-__device__ __forceinline__ void segment_advance(int p, int T, int nrows, int& q, int& oq) {
-  while (q + 1 < nrows && oq + (T - q) <= p) {
-    oq += T - q;
-    ++q;
-  }
-}
-
-// candidate column of entry p in row q (row start oq), clamped to the group's
-// column records
-__device__ __forceinline__ int segment_col(int p, int T, int q, int oq) { return min(max(q + (p - oq), q), T - 1); }
-
-// Two entries (rows qa, qb; candidate columns ta, tb) of a row group's segment
-// from the group's records (bases are wave-uniform; offsets are 32-bit). The two are computed side by side with
-// no branch between them, so that their loads are in flight together; the
-// second contribution (both specs of the row and of the column on the same
-// two Elems, a few entries in a hundred) follows.
-struct EntryRecs {  // the column and row records of two entries
-  uint4 ra, rb;
-  uint2 rpa, rpb;
-};
-
-__device__ __forceinline__ EntryRecs load_recs2(const uint4* __restrict__ col_g, const uint2* __restrict__ row_g,
-                                                int qa, int ta, int qb, int tb) {
-  EntryRecs r;
-  r.ra = ld32(col_g, unsigned(ta));
-  r.rb = ld32(col_g, unsigned(tb));
-  r.rpa = ld32(row_g, unsigned(qa));
-  r.rpb = ld32(row_g, unsigned(qb));
-  return r;
-}
-
-__device__ __forceinline__ void flat_entry2(const EntryRecs& rec, const double* __restrict__ coef_g,
-                                            const double* __restrict__ lib, unsigned tab, int& ca, double& cca,
-                                            double& l2a, int& cb, double& ccb, double& l2b) {
-  const uint4 ra = rec.ra, rb = rec.rb;
-  const uint2 rpa = rec.rpa, rpb = rec.rpb;
-  ca = int(ra.x);
-  cb = int(rb.x);
-  flat_contrib(lib, tab, coef_g, ra.w & 0xffu, ra.y, rpa, cca, l2a);
-  flat_contrib(lib, tab, coef_g, rb.w & 0xffu, rb.y, rpb, ccb, l2b);
-  if (ra.z != ~0u) {
-    double cc1, l21;
-    flat_contrib(lib, tab, coef_g, (ra.w >> 8) & 0xffu, ra.z, rpa, cc1, l21);
-    cca += cc1;
-    l2a += l21;
-  }
-  if (rb.z != ~0u) {
-    double cc1, l21;
-    flat_contrib(lib, tab, coef_g, (rb.w >> 8) & 0xffu, rb.z, rpb, cc1, l21);
-    ccb += cc1;
-    l2b += l21;
-  }
-}
-
 // Entry j of a chunk in the stored precision P, as three (four for FP32R)
 // coalesced, non-temporal stores; FP32R splits each value into its FP32 value
 // and 16-bit residual (fp32r.hpp)
@@ -1554,158 +1510,336 @@ __device__ __forceinline__ void store_entry(int* __restrict__ col_out, typename 
   }
 }
 
-// Streaming fill: the CSR is cut into chunks of w.chunk consecutive entries
-// (the size the layout scan used: Store<P>::kChunk, or the one tuned for the
-// Domain); wavefront v takes chunks v, v + waves, ..., so that the wavefronts
-// work on neighbouring chunks at any time and share each row group's records
-// in L2 (one contiguous range per wavefront, with no such sharing, ran 2.5-4x
-// slower). For each row group a chunk meets, the
-// wavefront stages the group's source records in LDS and writes the entries
-// with consecutive lanes on consecutive entries (coalesced, non-temporal
-// stores), reading the group's column and row records and the Gram library (a
-// per-block LDS copy when it fits). Entries of block-path groups are left to
-// k_fill_large. kACurlCurl / kBCurlCurl: A and B take the CurlCurl values
-// (else L2Inner); P: the stored precision (Store<P>; the arithmetic is FP64
-// in every precision, values are rounded once at the store).
-template <bool kLibInLds, bool kACurlCurl, bool kBCurlCurl, int P, int kSmall>
-__global__ void __launch_bounds__((FillShape<P, kSmall>::kBlock), kFillWavesPerSimd)
-    k_fill_flat(Work w, LibShape L, FillOut o) {
+// A row of a fill batch, in LDS: where its column records are (the index of the
+// record that an entry 0 of the chunk would have, from the records of the chunk's
+// first group; kLargeRow for a row of a block-path group, whose entries are not
+// the streaming fill's), shifted left by kSrcBits beside the first of its group's
+// sources in FillShared::src; and its parts of the library offsets by variant
+// (bit 0 the source is an ancestor, bit 1 the spec is on the group's second Elem).
+struct FillRow {
+  int at_src;
+  int pad;
+  uint2 var[4];
+};
+constexpr int kBatchRows = 32;
+constexpr int kBatchSrc = kWS;       // sources of a batch's groups: those of any one group fit
+constexpr int kSrcBits = 5;
+constexpr int kBatchEntries = 1024;  // entries of a batch at most (bits of its row bitmap)
+constexpr int kMaxChunk = 4096;
+constexpr int kLargeRow = -0x7fffffff - 1;
+// a chunk meets at most kMaxChunk + 1 groups, so a record index fits beside the source
+static_assert(kBatchSrc <= 1 << kSrcBits && (kMaxChunk + 2) * kWC < 1 << (31 - kSrcBits), "FillRow::at_src");
+
+// a wavefront's LDS of the streaming fill
+struct FillShared {
+  double4 src[kBatchSrc * kCoef / 4];
+  FillRow row[kBatchRows];
+  unsigned long long starts[kBatchEntries / kWave];  // bit p: a row starts at entry p + 1
+  int src_of[kBatchSrc];  // record of each source
+};
+
+// half of a source record, from its L2Inner prefactor on
+struct __attribute__((aligned(16))) SourceTail {
+  double cb;
+  unsigned x, y;
+};
+
+// Rounds of the streaming fill: a block takes kFillBlock / kWave consecutive
+// chunks at a time, one for each of its wavefronts, in the order in which the
+// blocks ask for them (w.ticket). So the entries that are being written at any
+// time lie close together, which the memory wants: a write-only probe of the three
+// arrays (87 M entries, 1.74 GB) took 285 us with rounds of 16 x 512 entries taken
+// by ticket, and 315-330 us with the same chunks dealt out in advance, whether to
+// resident blocks or block by block. A ticket costs 12 ns (one address, beyond the XCDs'
+// L2 caches), so rounds of less than about 16 x 256 entries are bound by it.
+// A block's first round is its own number. The first wavefront of a block to begin
+// its round k asks for round k + 2 once it has seen the ticket of round k + 1 (so
+// a block's tickets ascend, and the first one past the end is its last), and
+// passes the answer on when its chunk is written. kRing tickets are kept, and a barrier every
+// kRing / 2 rounds keeps a wavefront from falling behind the ring.
+constexpr int kRing = 64;
+struct FillRounds {
+  unsigned long long ring[kRing];  // round + 1 << 32 | ticket
+  int claimed;                     // rounds asked for
+};
+
+// One contribution to an entry: c and y the column's parts (col_contrib), row
+// its row, src the sources of its group.
+__device__ __forceinline__ void fill_contrib(const double* __restrict__ lib, const char* __restrict__ src,
+                                             const FillRow& row, unsigned c, unsigned y, double& cc, double& l2) {
+  const uint2 v = *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(row.var) + (c & 0x18u));
+  const char* s = src + (c & 0x7e0u);
+  const unsigned dr = v.y & 1u;
+  const double ca = *reinterpret_cast<const double*>(s + 8u * dr);
+  const SourceTail h = *reinterpret_cast<const SourceTail*>(s + 16);
+  const unsigned ix = h.x + (c >> 16) + unsigned(int(v.x << 16) >> 16);
+  const unsigned iy = h.y + y + unsigned(int(v.x) >> 16);
+  auto at = [&](unsigned o) { return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(lib) + o); };
+  const double fx = at(ix), fy = at(iy);
+  cc = ca * fx * fy;
+  // L2Inner (UU, VV only)
+  const double l2v = (h.cb * at(ix + (v.y & 0xfff8u))) * at(iy + (v.y >> 16));
+  l2 = ((c >> 5) & 1u) == dr ? l2v : 0.0;
+}
+
+// Streaming fill: the CSR is cut into chunks of w.chunk consecutive entries, which
+// the blocks take in rounds (FillRounds), a chunk for each wavefront.
+// A chunk is worked through in batches of up to kBatchRows rows: lane l prepares
+// row l of the batch (its start, from the group's segment, which is also its row
+// pointer; its parts of the library offsets), the sources of the batch's groups are
+// staged in LDS, and the rows' starts go into a bitmap. The batch's entries are then
+// written kWave at a time, whatever rows and groups they belong to: an entry's row
+// is the number of starts before it, its column record is the row's first one plus
+// its distance from the row's start.
+// Where its rows allow it a batch ends on a multiple of kWave entries, so that the
+// stores cover whole cache lines: with the groups taken one after another, the
+// stores of a group that starts inside a line wrote parts of lines (a write-only
+// probe of the three arrays took 175 us with its stores three entries off a line
+// and 100 us on it, 25.7 M entries), and small groups left most lanes idle.
+// kACurlCurl / kBCurlCurl: A and B take the CurlCurl values (else L2Inner); P:
+// the stored precision (Store<P>; the arithmetic is FP64 in every precision,
+// values are rounded once at the store).
+template <bool kLibInLds, bool kACurlCurl, bool kBCurlCurl, int P>
+__global__ void __launch_bounds__(kFillBlock, kFillWavesPerSimd) k_fill_flat(Work w, LibShape L, FillOut o) {
   using VA = typename Store<P>::A;
   using VB = typename Store<P>::B;
   if (*w.err) return;
-  // the source records of the row group being written, per wavefront
-  __shared__ double4 src_lds[FillShape<P, kSmall>::kBlock / kWave][kWS * kCoef / 4];
+  __shared__ FillShared shared[kFillBlock / kWave];
+  __shared__ FillRounds rounds;
   // the block's copy of the Gram library (when it fits)
-  __shared__ double lib_lds[kLibInLds ? FillShape<P, kSmall>::kLibLds : 1];
+  __shared__ double lib_lds[kLibInLds ? kFillLibLds : 1];
   const long long nnz = w.row_ptr[w.n_dofs];
   if (nnz > o.capacity) return;  // the host grows the buffers and runs the fill again
   if (kLibInLds) {
     const int n_lib = (L.nr + L.nr_v) * L.range_stride;
     for (int i = threadIdx.x; i < n_lib; i += blockDim.x) lib_lds[i] = w.lib[i];
-    __syncthreads();
   }
   const int lane = threadIdx.x % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(int((blockIdx.x * blockDim.x + threadIdx.x) / kWave));
-  const int waves = __builtin_amdgcn_readfirstlane(int(gridDim.x) * (FillShape<P, kSmall>::kBlock / kWave));
-  const long long chunk = w.chunk;  // the layout scan's chunk size (default or tuned per Domain)
+  FillShared& S = shared[threadIdx.x / kWave];
+  const long long chunk = w.chunk;
   const long long n_chunks = min((nnz + chunk - 1) / chunk, w.chunk_cap);
+  constexpr int kWaves = kFillBlock / kWave;
+  const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
+  auto answer = [&](int k, int t) {  // one lane
+    __hip_atomic_store(&rounds.ring[k % kRing], ((unsigned long long)unsigned(k + 1) << 32) | (gridDim.x + unsigned(t)),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  for (int i = threadIdx.x; i < kRing; i += blockDim.x) rounds.ring[i] = i == 0 ? (1ull << 32) | blockIdx.x : 0ull;
+  if (threadIdx.x == 0) rounds.claimed = 2;
+  __syncthreads();
+  if (threadIdx.x == 0) answer(1, atomicAdd(w.ticket, 1));
+  // this wavefront's chunk of the block's round k (past the last chunk at the end)
+  auto take = [&](int k) -> long long {
+    unsigned long long v;
+    while (true) {
+      v = __hip_atomic_load(&rounds.ring[k % kRing], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (__builtin_amdgcn_readfirstlane(int(v >> 32)) == k + 1) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    return (long long)unsigned(__builtin_amdgcn_readfirstlane(int(v))) * kWaves + wid;
+  };
   const double* __restrict__ lib = kLibInLds ? lib_lds : w.lib;
-  const unsigned tab = unsigned(L.tab);
-  // per-group values are wave-uniform: they come through scalar loads and stay
-  // in scalar registers (with the record bases). Loading each chunk's first row
-  // group one chunk ahead was measured 2-3 % slower.
-  for (long long ch = wave; ch < n_chunks; ch += waves) {
-    const long long pbase = ch * chunk;
+  const int tab = L.tab;
+  // lanes l and l + kBatchRows work on row l of a batch: the first on its spec on
+  // the group's first Elem, the other on the one on its second
+  const int row = lane % kBatchRows, k = lane / kBatchRows;
+  const bool lead = k == 0;  // one lane a row in what counts rows
+  // what the next batch's rows need is loaded while the entries of the batch
+  // before are written: their groups and specs, then the groups' headers
+  int g_ahead = 1;
+  unsigned spec_ahead = 0u;
+  int4 hdr_ahead = make_int4(0, 0, 0, 0);
+  long long seg_ahead = 0;
+  auto load_rows = [&](int r) {
+    if (r + (long long)row < w.n_dofs) {
+      g_ahead = w.dof_grp[r + row];
+      spec_ahead = reinterpret_cast<const unsigned*>(w.meta_row)[2LL * (r + row) + k];
+    }
+  };
+  auto load_groups = [&]() {
+    hdr_ahead = w.meta_hdr[g_ahead - 1];
+    seg_ahead = w.seg_start[g_ahead - 1];
+  };
+  long long ch_next = take(0);
+  int r = ch_next < n_chunks ? ld_const(w.chunk_first, ch_next) : 0;  // the batch's first row, which holds entry `pos`
+  load_rows(r);
+  load_groups();
+  for (int round = 0;; ++round) {
+    const long long ch = ch_next;
+    if (ch - wid >= n_chunks) break;  // the block's last round (every wavefront's)
+    if (round % (kRing / 2) == kRing / 2 - 1) __syncthreads();
+    ch_next = take(round + 1);
+    const bool asks = lane == 0 && atomicMax(&rounds.claimed, round + 3) < round + 3;
+    int asked = 0;
+    if (asks) asked = atomicAdd(w.ticket, 1);
+    if (ch >= n_chunks) {
+      if (asks) answer(round + 2, asked);
+      continue;
+    }
+    const long long pbase = uniform(ch * chunk);
     const int len = int(min(chunk, nnz - pbase));
-    const long long pb = uniform(pbase);
-    int* __restrict__ col_out = o.col + pb;
-    VA* __restrict__ a_out = static_cast<VA*>(o.aval) + pb;
-    VB* __restrict__ b_out = static_cast<VB*>(o.bval) + pb;
-    unsigned* __restrict__ r_out = Store<P>::kRes ? o.res + pb : nullptr;
-    int g = ld_const(w.chunk_first, ch);
-    int j0 = 0;
-    while (j0 < len) {
-      const long long S = ld_const(w.seg_start, g), S1 = ld_const(w.seg_start, g + 1);
-      const int j1 = int(min((long long)len, S1 - pbase));
-      const int4 hdr = ld_const(w.meta_hdr, g);
-      if (hdr.x > 0) {
-        const int T = hdr.x, nrows = hdr.y;
-        const int off = int(pbase - S);  // segment position of chunk entry 0
-        const float bq = 2.0f * float(T) + 1.0f;
-        const uint4* col_g = w.meta_col + (size_t)g * kWC;
-        const uint2* row_g = w.meta_row + hdr.w;  // the group's rows are DoFs hdr.w, hdr.w + 1, ...
-        // two entries per lane and iteration; past the end of the group's
-        // part of the chunk the second one repeats the first and is not stored.
-        // Each lane finds the row of its first entry from the root and then
-        // follows its entries (64 apart) row by row. The rows and columns are
-        // clamped into the group's records, so a lane past the part's end
-        // loads in bounds.
-        int qa, oqa;
-        segment_row(j0 + lane + off, T, nrows, bq, qa, oqa);
-        int j = j0 + lane;
-        bool second = j + kWave < j1;
-        int qb = qa, oqb = oqa;
-        {
-          const int pa = j + off, pb = (second ? j + kWave : j) + off;
-          segment_advance(pa, T, nrows, qa, oqa);
-          qb = qa;
-          oqb = oqa;
-          segment_advance(pb, T, nrows, qb, oqb);
-        }
-        // the first iteration's records are loaded before the source records
-        // are staged, so that the two loads are in flight together
-        EntryRecs rec = load_recs2(col_g, row_g, qa, segment_col(j + off, T, qa, oqa), qb,
-                                   segment_col((second ? j + kWave : j) + off, T, qb, oqb));
-        double4* stage = src_lds[threadIdx.x / kWave];
-        const double4* src_g = reinterpret_cast<const double4*>(w.meta_coef + (size_t)g * kWS * kCoef);
-        for (int i = lane; i < hdr.z * (kCoef / 4); i += kWave) stage[i] = src_g[i];
-        wave_sync();
-        const double* coef_g = reinterpret_cast<const double*>(stage);
-        while (j < j1) {
-          int c0, c1;
-          double cc0, l20, cc1, l21;
-          flat_entry2(rec, coef_g, lib, tab, c0, cc0, l20, c1, cc1, l21);
-          store_entry<P>(col_out, a_out, b_out, r_out, unsigned(j), c0, kACurlCurl ? cc0 : l20,
-                         kBCurlCurl ? cc0 : l20);
-          if (second)
-            store_entry<P>(col_out, a_out, b_out, r_out, unsigned(j + kWave), c1, kACurlCurl ? cc1 : l21,
-                           kBCurlCurl ? cc1 : l21);
-          j += 2 * kWave;
-          if (j >= j1) break;
-          qa = qb;
-          oqa = oqb;
-          second = j + kWave < j1;
-          const int pa = j + off, pb = (second ? j + kWave : j) + off;
-          segment_advance(pa, T, nrows, qa, oqa);
-          qb = qa;
-          oqb = oqa;
-          segment_advance(pb, T, nrows, qb, oqb);
-          rec = load_recs2(col_g, row_g, qa, segment_col(pa, T, qa, oqa), qb, segment_col(pb, T, qb, oqb));
-        }
-        wave_sync();  // every lane is done with the staged records
+    const int r_chunk = ch_next < n_chunks ? ld_const(w.chunk_first, ch_next) : r;  // the next chunk's
+    int* __restrict__ col_out = o.col + pbase;
+    VA* __restrict__ a_out = static_cast<VA*>(o.aval) + pbase;
+    VB* __restrict__ b_out = static_cast<VB*>(o.bval) + pbase;
+    unsigned* __restrict__ r_out = Store<P>::kRes ? o.res + pbase : nullptr;
+    int g0 = 0;
+    const uint4* __restrict__ col_g = nullptr;
+    int pos = 0;
+    while (pos < len) {
+      // the row's entries are [s, end) of the chunk
+      const long long rr = r + (long long)row;
+      const bool valid = rr < w.n_dofs;
+      const int g = g_ahead - 1;
+      const int4 hdr = hdr_ahead;
+      const bool large = valid && hdr.x <= 0;
+      int s = len, end = len, q = 0, n_src = 0;
+      bool first = false;
+      if (pos == 0) {  // the group of the chunk's first row
+        g0 = __builtin_amdgcn_readfirstlane(g);
+        col_g = w.meta_col + (long long)g0 * kWC;
       }
-      j0 = j1;
-      ++g;
+      if (large) {  // the layout scan wrote its row pointers
+        s = int(w.row_ptr[rr] - pbase);
+        end = s + int(w.row_len[rr]);
+      } else if (valid) {
+        q = int(rr) - hdr.w;
+        s = int(seg_ahead - pbase) + int(__umul24(unsigned(q), unsigned(2 * hdr.x - q + 1)) >> 1);
+        end = s + hdr.x - q;
+        n_src = hdr.z;
+        first = q == 0 || row == 0;
+      }
+      S.row[row].var[2 * k] = row_variant(spec_ahead, false, tab);
+      S.row[row].var[2 * k + 1] = row_variant(spec_ahead, true, tab);
+      const int src_end = wave_incl_scan(lead && first ? n_src : 0, lane);  // sources up to and with the row's group
+      // the batch: entries [pos, limit), pieces of kWave from the multiple at or below pos
+      const int at0 = pos & ~(kWave - 1);
+      int limit = min(min(len, at0 + kBatchEntries), __builtin_amdgcn_readlane(end, kBatchRows - 1));
+      const unsigned long long over = __ballot(lead && valid && src_end > kBatchSrc);
+      if (over) limit = min(limit, __builtin_amdgcn_readlane(s, __builtin_ctzll(over)));
+      if (limit < len && (limit & ~(kWave - 1)) > pos) limit &= ~(kWave - 1);
+      if (limit <= pos) {  // the first row holds entry pos: the layout disagrees with itself
+        if (lane == 0) set_err(w.err, kErrView);
+        break;
+      }
+      const bool in = lead && valid && s < limit;
+      if (in && !large && s >= pos) w.row_ptr[rr] = pbase + s;
+      if (in)
+        S.row[row].at_src =
+            large ? kLargeRow
+                  : int((unsigned((g - g0) * kWC + col_slot(g, end - s + q) + q - s) << kSrcBits) |
+                        unsigned(src_end - n_src));
+      if (lane < kBatchEntries / kWave) S.starts[lane] = 0;
+      if (in && first)
+        for (int k = 0; k < n_src; ++k) S.src_of[src_end - n_src + k] = g * kWS + src_slot(g, n_src) + k;
+      wave_sync();
+      const unsigned long long taken = __ballot(in && first);
+      const int total_src = taken ? __builtin_amdgcn_readlane(src_end, 63 - __builtin_clzll(taken)) : 0;
+      for (int i = lane; i < total_src * (kCoef / 4); i += kWave)
+        S.src[i] = reinterpret_cast<const double4*>(w.meta_coef)[(long long)S.src_of[i / (kCoef / 4)] * (kCoef / 4) +
+                                                                 i % (kCoef / 4)];
+      r += __popcll(__ballot(lead && valid && end <= limit));  // past the rows that end in this batch
+      if (limit == len) r = r_chunk;
+      load_rows(r);
+      if (in && lane > 0) {
+        const int bit = s - at0 - 1;
+        atomicOr(&S.starts[bit / kWave], 1ull << (bit % kWave));
+      }
+      wave_sync();
+      int before = 0;  // rows that start in the pieces before
+      // an entry's row, column record and contributions
+      auto find = [&](unsigned long long m) -> const FillRow& {
+        const int i = int(__builtin_amdgcn_mbcnt_hi(unsigned(m >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(m), before)));
+        before += __popcll(m);
+        return S.row[i];
+      };
+      auto record = [&](const FillRow& row, int p) { return ld32(col_g, unsigned((row.at_src >> kSrcBits) + p)); };
+      auto contrib = [&](const FillRow& row, unsigned c, unsigned y, double& cc, double& l2) {
+        const unsigned src = unsigned(row.at_src) % (1u << kSrcBits) * unsigned(kCoef * sizeof(double));
+        fill_contrib(lib, reinterpret_cast<const char*>(S.src) + src, row, c, y, cc, l2);
+      };
+      auto second = [&](const FillRow& row, const uint4& rec, double& cc, double& l2) {
+        double c1, l1;
+        contrib(row, rec.z, rec.w >> 16, c1, l1);
+        cc += c1;
+        l2 += l1;
+      };
+      auto starts = [&](int j) { return (unsigned long long)uniform((long long)S.starts[(j - at0) / kWave]); };
+      if (__ballot(large && in) == 0) {
+        // two pieces at a time, computed side by side with no branch between
+        // them, the records of the next two loading meanwhile (ahead of this
+        // two's stores, so that waiting for them waits for no store); lanes
+        // outside the batch repeat its first or last entry and store nothing
+        struct Pair {
+          const FillRow *ra, *rb;
+          uint4 ca, cb;
+        };
+        auto load = [&](int j) {
+          Pair n;
+          const int p0 = j + lane;
+          n.ra = &find(starts(j));
+          n.rb = &find(starts(min(j + kWave, at0 + kBatchEntries - kWave)));
+          n.ca = record(*n.ra, min(max(p0, pos), limit - 1));
+          n.cb = record(*n.rb, min(p0 + kWave, limit - 1));
+          return n;
+        };
+        Pair x = load(at0);
+        load_groups();
+        for (int j = at0; j < limit; j += 2 * kWave) {
+          const Pair c = x;
+          if (j + 2 * kWave < limit) x = load(j + 2 * kWave);
+          const int p0 = j + lane;
+          double cca, l2a, ccb, l2b;
+          contrib(*c.ra, c.ca.y, c.ca.w & 0xffffu, cca, l2a);
+          contrib(*c.rb, c.cb.y, c.cb.w & 0xffffu, ccb, l2b);
+          // both specs of the row and of the column on the same two Elems: a few entries in a hundred
+          if (c.ca.z != ~0u) second(*c.ra, c.ca, cca, l2a);
+          if (c.cb.z != ~0u) second(*c.rb, c.cb, ccb, l2b);
+          if (p0 >= pos && p0 < limit)
+            store_entry<P>(col_out, a_out, b_out, r_out, unsigned(p0), int(c.ca.x), kACurlCurl ? cca : l2a,
+                           kBCurlCurl ? cca : l2a);
+          if (p0 + kWave < limit)
+            store_entry<P>(col_out + kWave, a_out + kWave, b_out + kWave, r_out + (Store<P>::kRes ? kWave : 0),
+                           unsigned(p0), int(c.cb.x), kACurlCurl ? ccb : l2b, kBCurlCurl ? ccb : l2b);
+        }
+      } else {
+        load_groups();
+        for (int j = at0; j < limit; j += kWave) {
+          const int p = j + lane;
+          const FillRow& ra = find(starts(j));
+          if (p >= pos && p < limit && ra.at_src != kLargeRow) {
+            const uint4 ca = record(ra, p);
+            double cca, l2a;
+            contrib(ra, ca.y, ca.w & 0xffffu, cca, l2a);
+            if (ca.z != ~0u) second(ra, ca, cca, l2a);
+            store_entry<P>(col_out, a_out, b_out, r_out, unsigned(p), int(ca.x), kACurlCurl ? cca : l2a,
+                           kBCurlCurl ? cca : l2a);
+          }
+        }
+      }
+      pos = limit;
+      wave_sync();  // every lane is done with the batch's LDS
     }
-  }
-  // row pointers of the streaming-fill groups' rows, after the entries (the
-  // fill reads none of them; written last they overlap other wavefronts'
-  // final chunks): row q of group g starts q T - q (q - 1) / 2 entries into
-  // the group's segment (the layout scan writes those of block-path groups)
-  for (long long r = blockIdx.x * (long long)blockDim.x + threadIdx.x; r < w.n_dofs;
-       r += (long long)gridDim.x * blockDim.x) {
-    const int g = w.dof_grp[r] - 1;
-    const int T = w.meta_hdr[g].x;
-    if (T > 0) {
-      const long long q = r - w.g_start[g];
-      w.row_ptr[r] = w.seg_start[g] + q * T - q * (q - 1) / 2;
-    }
+    if (asks) answer(round + 2, asked);  // the answer came while the chunk was written
   }
 }
 
-// one instance per library placement, integral pair, stored precision and shape
-template <bool kLibInLds, int P, int kSmall>
+// one instance per library placement, integral pair and stored precision
+template <bool kLibInLds, int P>
 void launch_fill_lib(bool a_cc, bool b_cc, unsigned grid, hipStream_t st, const Work& w, const LibShape& L,
                      const FillOut& o) {
-  constexpr int B = FillShape<P, kSmall>::kBlock;
-  if (a_cc && !b_cc) k_fill_flat<kLibInLds, true, false, P, kSmall><<<grid, B, 0, st>>>(w, L, o);
-  else if (!a_cc && b_cc) k_fill_flat<kLibInLds, false, true, P, kSmall><<<grid, B, 0, st>>>(w, L, o);
-  else if (a_cc) k_fill_flat<kLibInLds, true, true, P, kSmall><<<grid, B, 0, st>>>(w, L, o);
-  else k_fill_flat<kLibInLds, false, false, P, kSmall><<<grid, B, 0, st>>>(w, L, o);
+  constexpr int B = kFillBlock;
+  if (a_cc && !b_cc) k_fill_flat<kLibInLds, true, false, P><<<grid, B, 0, st>>>(w, L, o);
+  else if (!a_cc && b_cc) k_fill_flat<kLibInLds, false, true, P><<<grid, B, 0, st>>>(w, L, o);
+  else if (a_cc) k_fill_flat<kLibInLds, true, true, P><<<grid, B, 0, st>>>(w, L, o);
+  else k_fill_flat<kLibInLds, false, false, P><<<grid, B, 0, st>>>(w, L, o);
 }
-
-// the small shape exists for the precisions whose own shape is larger
-template <int P>
-constexpr bool kHasSmall = Store<P>::kBlock > 512;
 
 template <int P>
 void launch_fill_prec(int place, bool a_cc, bool b_cc, unsigned grid, hipStream_t st, const Work& w,
                       const LibShape& L, const FillOut& o) {
-  if constexpr (kHasSmall<P>) {
-    if (place == kPlaceLdsSmall) return launch_fill_lib<true, P, 1>(a_cc, b_cc, grid, st, w, L, o);
-  }
-  if (place != kPlaceGlobal) launch_fill_lib<true, P, 0>(a_cc, b_cc, grid, st, w, L, o);
-  else launch_fill_lib<false, P, 0>(a_cc, b_cc, grid, st, w, L, o);
+  if (place != kPlaceGlobal) launch_fill_lib<true, P>(a_cc, b_cc, grid, st, w, L, o);
+  else launch_fill_lib<false, P>(a_cc, b_cc, grid, st, w, L, o);
 }
 
 void launch_fill(int place, bool a_cc, bool b_cc, unsigned grid, hipStream_t st, const Work& w, const LibShape& L,
@@ -1719,30 +1853,14 @@ void launch_fill(int place, bool a_cc, bool b_cc, unsigned grid, hipStream_t st,
   }
 }
 
-template <int P>
-long long lib_lds_cap(int place) {
-  if constexpr (kHasSmall<P>) {
-    if (place == kPlaceLdsSmall) return FillShape<P, 1>::kLibLds;
-  }
-  return place == kPlaceLds ? Store<P>::kLibLds : 0;
-}
-
-// the library fits the fill's LDS copy of a placement (kPlaceGlobal always
-// fits; kPlaceLdsSmall only for the precisions that have the small shape)
-bool place_fits(int precision, int place, long long lib_n) {
-  if (place == kPlaceGlobal) return true;
-  switch (precision) {
-    case FEM2D_PRECISION_FP32: return lib_n <= lib_lds_cap<FEM2D_PRECISION_FP32>(place);
-    case FEM2D_PRECISION_FP32R: return lib_n <= lib_lds_cap<FEM2D_PRECISION_FP32R>(place);
-    default: return lib_n <= lib_lds_cap<FEM2D_PRECISION_FP64>(place);
-  }
-}
+// the library fits the fill's LDS copy of a placement (kPlaceGlobal always fits)
+bool place_fits(int place, long long lib_n) { return place == kPlaceGlobal || lib_n <= kFillLibLds; }
 
 // the placement an assembly uses: the tuned one, else the LDS copy when the
 // library fits it
-int fill_place(int precision, int tuned, long long lib_n) {
-  if (tuned >= 0 && place_fits(precision, tuned, lib_n)) return tuned;
-  return place_fits(precision, kPlaceLds, lib_n) ? kPlaceLds : kPlaceGlobal;
+int fill_place(int tuned, long long lib_n) {
+  if (tuned >= 0 && place_fits(tuned, lib_n)) return tuned;
+  return place_fits(kPlaceLds, lib_n) ? kPlaceLds : kPlaceGlobal;
 }
 
 // ---------------------------------------------------------------------------
@@ -2305,7 +2423,7 @@ struct fem2d_ctx {
   int count_grid = 0;  // resident blocks of the wave kernels on this device
   // resident blocks of the streaming fill per stored precision, with the library in
   // global memory / in LDS
-  int fill_grid[kPrecisions][3] = {};  // resident blocks of the fill per precision and FillPlace
+  int fill_grid[kPrecisions][2] = {};  // resident blocks of the fill per precision and FillPlace
   bool use_graphs = true;
   bool autotune = true;  // time the fill's chunk sizes on a Domain's first assembly
   int fill_chunk = 0;     // fill chunk size forced for every assembly (0: tuned or default)
@@ -2648,6 +2766,7 @@ int bind_work(const fem2d_device_domain* dd, int nu, int nv, int basis, Bind&& b
       (rc = bind(k++, N1, &w.large_list)) || (rc = bind(k++, N1, &w.is_large)))
     return rc;
   w.n_large = w.err + 1;
+  w.ticket = w.err + 2;
   const size_t G1 = size_t(std::max(1LL, dd->n_groups));
   w.meta_cap = int(G1);
   if ((rc = bind(k++, G1, &w.meta_hdr)) || (rc = bind(k++, G1 * kWS * kCoef, &w.meta_coef)) ||
@@ -2665,6 +2784,7 @@ int bind_work(const fem2d_device_domain* dd, int nu, int nv, int basis, Bind&& b
   L.nv = nv;
   L.basis = basis;
   a.lib_n = (long long)(L.nr + L.nr_v) * kKinds * L.p1 * L.p1;
+  w.lib_tab = L.tab;
   w.lib_range_stride = L.range_stride;
   w.lib_nr = L.nr;
   w.lib_nr_v = L.nr_v;
@@ -2751,7 +2871,7 @@ int launch_prep(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, long long* st
 // buffers it writes nothing)
 int launch_stream_fill(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, const FillOut& o) {
   const int pi = o.precision;
-  const int place = fill_place(o.precision, a.lib_lds, a.lib_n);
+  const int place = fill_place(a.lib_lds, a.lib_n);
   launch_fill(place, o.a_is_cc != 0, o.b_is_cc != 0, unsigned(ctx->fill_grid[pi][place]), st, a.w, a.L, o);
   HIP_TRY_AT(hipGetLastError(), "after the fill kernel");
   return FEM2D_OK;
@@ -2770,18 +2890,10 @@ int launch_large_fill(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, const F
 template <int P>
 int fill_grids(fem2d_ctx* ctx) {
   int per_cu = 0;
-  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fill_flat<false, true, false, P, 0>,
-                                                       Store<P>::kBlock, 0));
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fill_flat<false, true, false, P>, kFillBlock, 0));
   ctx->fill_grid[P][kPlaceGlobal] = std::max(1, per_cu) * ctx->n_cu;
-  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fill_flat<true, true, false, P, 0>,
-                                                       Store<P>::kBlock, 0));
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fill_flat<true, true, false, P>, kFillBlock, 0));
   ctx->fill_grid[P][kPlaceLds] = std::max(1, per_cu) * ctx->n_cu;
-  ctx->fill_grid[P][kPlaceLdsSmall] = ctx->fill_grid[P][kPlaceLds];
-  if constexpr (kHasSmall<P>) {
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fill_flat<true, true, false, P, 1>,
-                                                         FillShape<P, 1>::kBlock, 0));
-    ctx->fill_grid[P][kPlaceLdsSmall] = std::max(1, per_cu) * ctx->n_cu;
-  }
   return FEM2D_OK;
 }
 
@@ -2801,7 +2913,7 @@ FillOut make_fill_out(int precision, int ai, int bi, long long capacity, int* co
 
 // chunk sizes the fill's autotuning times on a Domain's first assembly, each
 // placement and size timed kTuneReps times (the fastest launch counts)
-constexpr int kChunkCandidates[] = {128, 256, 512, 1024};
+constexpr int kChunkCandidates[] = {256, 512, 768};
 constexpr int kTuneReps = 5;
 
 // FEM2D_TUNE_VERBOSE=1 prints every tuning trial's time to stderr
@@ -2813,17 +2925,8 @@ bool tune_verbose() {
   return on;
 }
 
-// CSR entries per fill chunk for a stored precision (before any tuning)
-int chunk_of(int precision) {
-  switch (precision) {
-    case FEM2D_PRECISION_FP32: return Store<FEM2D_PRECISION_FP32>::kChunk;
-    case FEM2D_PRECISION_FP32R: return Store<FEM2D_PRECISION_FP32R>::kChunk;
-    default: return Store<FEM2D_PRECISION_FP64>::kChunk;
-  }
-}
-
-// w.chunk for a chunk size (0: the stored precision's default)
-void set_chunk(Work& w, int chunk, int precision) { w.chunk = chunk > 0 ? chunk : chunk_of(precision); }
+// w.chunk for a chunk size (0: the default)
+void set_chunk(Work& w, int chunk) { w.chunk = chunk > 0 ? chunk : kFillChunk; }
 
 // Host metadata of a device Domain that depends on the Elem tree only: the
 // sub-ranges of the Gram library (the position of each Elem inside each of its
@@ -3243,7 +3346,7 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
       return rc;
     const FillOut o = make_fill_out(precision, ai, bi, ctx->out_capacity, static_cast<int*>(ctx->out_col.p),
                                     ctx->out_a.p, ctx->out_b.p, static_cast<unsigned*>(ctx->out_r.p));
-    set_chunk(w, ctx->fill_chunk ? ctx->fill_chunk : dd->tuned_chunk[precision], precision);
+    set_chunk(w, ctx->fill_chunk ? ctx->fill_chunk : dd->tuned_chunk[precision]);
     w.chunk_cap = o.capacity / w.chunk + 1;
     if ((rc = slot(ctx, kChunkSlot, size_t(w.chunk_cap), &w.chunk_first))) return rc;
     const bool fill = o.capacity > 0;
@@ -3317,7 +3420,7 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
   dd->large_state = n_large > 0 ? 1 : 0;
   a.run_large = n_large > 0;  // the tuning trials below skip the block path's count when it has no group
   ctx->timing.fill_chunk = w.chunk;
-  ctx->timing.fill_lib_lds = fill_place(precision, a.lib_lds, a.lib_n);
+  ctx->timing.fill_lib_lds = fill_place(a.lib_lds, a.lib_n);
   if (ctx->autotune && !ctx->fill_chunk && dd->tuned_chunk[precision] == 0) {
     // the first assembly of this Domain in this precision: time the streaming
     // fill at each candidate chunk size and library placement (best of
@@ -3330,11 +3433,11 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
     // the repetitions are the outer loop, so that a drift of the GPU's clocks
     // over the trials favours no candidate
     for (int rep = 0; rep < kTuneReps; ++rep)
-      for (int place : {kPlaceLdsSmall, kPlaceLds, kPlaceGlobal}) {
-        if (!place_fits(precision, place, a.lib_n)) continue;
+      for (int place : {kPlaceLds, kPlaceGlobal}) {
+        if (!place_fits(place, a.lib_n)) continue;
         a.lib_lds = place;
         for (int c : kChunkCandidates) {
-          set_chunk(w, c, precision);
+          set_chunk(w, c);
           w.chunk_cap = o.capacity / w.chunk + 1;
           if ((rc = slot(ctx, kChunkSlot, size_t(w.chunk_cap), &w.chunk_first))) return rc;
           if ((rc = launch_prep(ctx, st, a, ctx->d_status, false))) return rc;
@@ -3417,7 +3520,7 @@ int fem2d_assemble_device_noalloc(fem2d_ctx* ctx, const fem2d_device_domain* dd,
   a.lib_lds = dd->tuned_lds[precision];
   Work& w = a.w;
   w.row_ptr = row_ptr;
-  set_chunk(w, ctx->fill_chunk ? ctx->fill_chunk : dd->tuned_chunk[precision], precision);
+  set_chunk(w, ctx->fill_chunk ? ctx->fill_chunk : dd->tuned_chunk[precision]);
   w.chunk_cap = capacity / w.chunk + 1;
   w.chunk_first = static_cast<int*>(carve(size_t(w.chunk_cap) * sizeof(int)));
   if (used > kScratchBytes) {
