@@ -24,7 +24,7 @@ dense GPU eigensolves of assembled GEPs (with LAPACK on the host beside them);
 beside it); `fields` the field evaluation over every leaf of the Domain; `sparse_eigensolve`
 the sparse shift-invert eigensolve of the workload's GEP near the TE10 cutoff;
 `other_workloads` the assembly of the hp-irregular (KOL, 1.78 M DoFs) and 256-guide
-configurations at full size, each with its fill roofline and tuned chunk size.
+configurations at full size, each with its fill roofline and chunk size.
 `cpu_baseline` times the oracle (the C++
 restatement of the reference algorithm) on a bounded sample of the same
 workload on the host cores. `mixed_precision` repeats the measurement with the values
@@ -48,7 +48,7 @@ METRIC = "GEP assembly nonzeros/s: mixed-prec vs FP64 GPU at stated rel err; CPU
 HBM_PEAK_GBS = 8000.0
 BYTES_PER_ENTRY = 20  # col (4) + A (8) + B (8)
 # the fill's Gram library placement (fem2d_timing.fill_lib_lds)
-FILL_PLACEMENT = {0: "global", 1: "lds", 2: "lds_small_blocks"}
+FILL_PLACEMENT = {0: "global", 1: "lds"}
 
 
 def build_workload(name: str):
@@ -189,7 +189,7 @@ def mixed_precision(dd, w, args, nnz: int, ms_fp64: float, fill_fp64_ms: float):
 
 def other_workload(name: str, steps: int = 10, warmup: int = 3):
     """Assembly throughput of another configuration at its full size: the timed graph replays,
-    the fill kernel kernel by kernel (its HBM roofline), and the chunk size the autotuning chose."""
+    the fill kernel kernel by kernel (its HBM roofline), and its chunk size."""
     import numpy as np
 
     import fem_2d_amd as F

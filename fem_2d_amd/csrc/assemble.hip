@@ -108,7 +108,7 @@ struct Store<FEM2D_PRECISION_FP32R> {
 // 152 us on 37.6 M in small groups).
 constexpr int kFillBlock = 1024;
 constexpr int kFillLibLds = 12288;
-constexpr int kFillChunk = 512;  // CSR entries per work item, before any tuning
+constexpr int kMaxChunk = 4096;  // CSR entries per work item (chunk) of the fill at most
 // placements of the fill's Gram library: global memory, or an LDS copy
 enum FillPlace { kPlaceGlobal = 0, kPlaceLds = 1 };
 constexpr int kFillWavesPerSimd = 4;
@@ -221,7 +221,9 @@ struct Work {
   int64_t* seg_start;  // [G+1] first CSR entry of each row group
   int* chunk_first;    // [chunk_cap] row holding the first entry of each chunk
   long long chunk_cap;
-  int chunk;           // CSR entries per chunk
+  int chunk;           // CSR entries per chunk forced by the caller (0: fill_chunk_of's)
+  int chunk_max;       // fill_chunk_of's upper bound for the stored precision
+  int fill_waves;      // wavefronts of the fill's launch
   long long n_dofs;
 };
 
@@ -487,6 +489,20 @@ __device__ __forceinline__ void pair_values(const double* __restrict__ lib, unsi
     if (pd == 0) l2 = cB[0] * fx * ld32(lib, iy + __umul24(unsigned(kTT), tab));
     else l2 = cB[1] * ld32(lib, ix + __umul24(unsigned(kTT), tab)) * fy;
   }
+}
+
+// a wave-uniform value loaded through the vector path, moved to a scalar register
+__device__ __forceinline__ long long uniform(long long x) {
+  const unsigned long long u = (unsigned long long)x;
+  return (long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(int(u >> 32)) << 32) |
+                     (unsigned)__builtin_amdgcn_readfirstlane(int(u & 0xffffffffu)));
+}
+
+// the value that lane l (wave-uniform) has
+__device__ __forceinline__ long long lane_value(long long x, int l) {
+  const unsigned long long v = (unsigned long long)x;
+  return (long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readlane(int(v >> 32), l) << 32) |
+                     (unsigned)__builtin_amdgcn_readlane(int(v & 0xffffffffu), l));
 }
 
 // ---------------------------------------------------------------------------
@@ -870,6 +886,29 @@ __device__ __forceinline__ void segment_row(int p, int T, int nrows, float bq, i
   q += up ? 1 : 0;
 }
 
+// CSR entries per chunk of the streaming fill: a multiple of kWave such that nnz
+// entries make whole rounds of one chunk a wavefront, in as few rounds as chunks of
+// max_chunk entries allow. A chunk costs a chain of dependent loads before its
+// first entry, so few large ones are faster (25.7 M entries, FP64: 256 entries
+// 113 us, 384 101, 512 100, 768 111; FP32: 512 87, 640 82, 768 84, 1024 85) until a
+// round leaves wavefronts idle (5.2 M entries: 320 51 us, 512 55, 1024 73). The
+// table of first rows (cap chunks) may demand larger ones.
+__host__ __device__ __forceinline__ int fill_chunk_of(long long nnz, long long cap, int waves, int max_chunk) {
+  const long long round = (long long)waves * max_chunk;
+  const long long rounds = nnz > round ? (nnz + round - 1) / round : 1;
+  long long c = (nnz + waves * rounds - 1) / (waves * rounds);
+  const long long least = (nnz + cap - 1) / cap;
+  if (c < least) c = least;
+  if (c < 1) c = 1;
+  return int((c + kWave - 1) / kWave * kWave);
+}
+// entries of the table of first rows for the chunks that fill_chunk_of makes of up to
+// `capacity` entries
+long long fill_chunk_cap(long long capacity, int waves, int max_chunk) { return capacity / max_chunk + waves + 1; }
+__device__ __forceinline__ int fill_chunk(const Work& w, long long nnz) {
+  return w.chunk ? w.chunk : fill_chunk_of(nnz, w.chunk_cap, w.fill_waves, w.chunk_max);
+}
+
 // First column record and first source record of row group g inside its slots of
 // kWC and kWS records. The slots are multiples of the memory channels' interleaving
 // apart and most groups fill a small part of them: with every group's records at
@@ -886,56 +925,17 @@ __device__ __forceinline__ int src_slot(int g, int n_src) {
 // of a streaming-fill group holds T - q entries, so the segment is
 // nrows T - nrows (nrows - 1) / 2 long; a block-path group sums the row
 // lengths its count kernel wrote. The exclusive sum is the segment's first
-// entry. The store writes the row of the first entry of each chunk of w.chunk
-// entries that starts inside the segment and, for a block-path group, row_ptr of
-// its rows (the streaming fill writes those of the other groups). The item past the
-// last group carries nnz and writes the call's status block (nnz, error bits,
-// block-path groups, row groups).
+// entry.
 struct GroupScan {
-  static constexpr int kRounds = 1;  // one group per thread: the store's chunk loop is the long part
+  static constexpr int kRounds = 1;
   Work w;
-  long long n_items;  // row groups the host sized the buffers for, plus one
-  long long* status;
-  __device__ long long seg_len(int g, int r0, int nrows, int4 hdr) const {
-    if (hdr.x > 0) return (long long)nrows * hdr.x - (long long)nrows * (nrows - 1) / 2;
-    long long len = 0;
-    for (int q = 0; q < nrows; ++q) len += w.row_len[r0 + q];
-    return len;
-  }
   __device__ long long load(long long g) const {
     if (*w.err || g >= n_groups_of(w)) return 0;
-    const int r0 = w.g_start[g];
-    return seg_len(int(g), r0, w.g_start[g + 1] - r0, w.meta_hdr[g]);
-  }
-  __device__ void store(long long g, long long excl, long long len) const {
-    w.seg_start[g] = excl;
-    const int n_groups = n_groups_of(w);
-    if (g == n_items - 1) {
-      w.row_ptr[w.n_dofs] = excl;
-      status[0] = excl;
-      status[1] = *w.err;
-      status[2] = *w.n_large;
-      status[3] = n_groups;
-    }
-    if (*w.err || g >= n_groups) return;  // an invalid view: the group records are not trustworthy
     const int4 hdr = w.meta_hdr[g];
-    const long long C = w.chunk;
-    long long c = (excl + C - 1) / C;
-    if (hdr.x <= 0) {  // a block-path group (the streaming fill writes the row pointers of the others)
-      const int r0 = w.g_start[g], nrows = w.g_start[g + 1] - r0;
-      long long at = excl;
-      for (int q = 0; q < nrows; ++q) {
-        w.row_ptr[r0 + q] = at;
-        at += w.row_len[r0 + q];
-        for (; c * C < at && c < w.chunk_cap; ++c) w.chunk_first[c] = r0 + q;
-      }
-      return;
-    }
-    for (; c * C < excl + len && c < w.chunk_cap; ++c) {
-      int q, oq;
-      segment_row(int(c * C - excl), hdr.x, hdr.y, 2.0f * float(hdr.x) + 1.0f, q, oq);
-      w.chunk_first[c] = hdr.w + q;
-    }
+    if (hdr.x > 0) return (long long)hdr.y * hdr.x - (long long)hdr.y * (hdr.y - 1) / 2;
+    long long len = 0;
+    for (int r = w.g_start[g]; r < w.g_start[g + 1]; ++r) len += w.row_len[r];
+    return len;
   }
 };
 
@@ -1133,6 +1133,106 @@ __global__ void __launch_bounds__(kBlock) k_scan_apply(long long n, Op op, const
   scan_apply_body(n, op, tile_sum, blockIdx.x, gridDim.x);
 }
 
+// Second pass of the CSR layout over n_items - 1 row groups (those that the host
+// sized the buffers for), one group a thread: the segments' first entries, the row
+// pointers of block-path groups (the streaming fill writes the others'), and the row
+// of the first entry of each of the fill's chunks that starts in the group's
+// segment (a group with many of them gets its whole wavefront). The item past the
+// last group carries nnz and writes the call's status block (nnz, error bits,
+// block-path groups, row groups). Without tile_sum (few groups) every block sums the
+// groups before its own, and `parts` blocks share a tile's chunks (94 groups of 3 700
+// entries: 13.8 us with one block, 5.2 with eight).
+__global__ void __launch_bounds__(kBlock) k_layout(Work w, long long n_items, const long long* tile_sum, int parts,
+                                                   long long* status) {
+  __shared__ long long s_wave[kWavesPerBlock], s_pre[kWavesPerBlock], s_all[kWavesPerBlock];
+  const GroupScan op{w};
+  const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+  const long long n_tiles = scan_tiles(n_items, 1);
+  const bool bad = *w.err != 0;  // an invalid view: the group records are not trustworthy
+  const int n_groups = n_groups_of(w);
+  const int part = int(blockIdx.x) % parts;  // the first writes what is written once
+  for (long long tile = blockIdx.x / parts; tile < n_tiles; tile += gridDim.x / parts) {
+    const long long g = tile * kBlock + threadIdx.x;
+    const long long len = g < n_items ? op.load(g) : 0;
+    const bool real = !bad && g < n_groups && g < n_items - 1;
+    const int4 hdr = real ? w.meta_hdr[g] : make_int4(0, 0, 0, 0);
+    long long pre = 0, all = 0;  // lengths of the tiles before this one and of all
+    if (tile_sum) {
+      for (long long t = threadIdx.x; t < n_tiles; t += kBlock) {
+        const long long x = tile_sum[t];
+        all += x;
+        pre += t < tile ? x : 0;
+      }
+    } else {
+      for (long long t = 0; t < n_tiles; ++t) {
+        const long long i = t * kBlock + threadIdx.x;
+        const long long x = t == tile ? len : i < n_items ? op.load(i) : 0;
+        all += x;
+        pre += t < tile ? x : 0;
+      }
+    }
+    long long incl = len;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const long long y = __shfl_up(incl, d, kWave);
+      if (lane >= d) incl += y;
+      pre += __shfl_xor(pre, d, kWave);
+      all += __shfl_xor(all, d, kWave);
+    }
+    if (lane == kWave - 1) s_wave[wid] = incl;
+    if (lane == 0) {
+      s_pre[wid] = pre;
+      s_all[wid] = all;
+    }
+    __syncthreads();
+    long long start = incl - len, nnz = 0;
+#pragma unroll
+    for (int v = 0; v < kWavesPerBlock; ++v) {
+      start += s_pre[v] + (v < wid ? s_wave[v] : 0);
+      nnz += s_all[v];
+    }
+    if (g < n_items && part == 0) w.seg_start[g] = start;
+    if (g == n_items - 1 && part == 0) {
+      w.row_ptr[w.n_dofs] = start;
+      status[0] = start;
+      status[1] = *w.err;
+      status[2] = *w.n_large;
+      status[3] = n_groups;
+    }
+    const long long C = fill_chunk(w, nnz);
+    // chunks [c, c1) start in the segment
+    long long c = (start + C - 1) / C, c1 = min((start + len + C - 1) / C, w.chunk_cap);
+    if (!real || (part > 0 && hdr.x <= 0)) c1 = c;
+    if (real && hdr.x <= 0 && part == 0) {  // a block-path group
+      long long at = start;
+      for (int r = w.g_start[g]; r < w.g_start[g + 1]; ++r) {
+        w.row_ptr[r] = at;
+        at += w.row_len[r];
+        for (; c < c1 && c * C < at; ++c) w.chunk_first[c] = r;
+      }
+    }
+    auto first_row = [](long long p, int4 h) {
+      int q, oq;
+      segment_row(int(p), h.x, h.y, 2.0f * float(h.x) + 1.0f, q, oq);
+      return h.w + q;
+    };
+    constexpr int kOwn = 16;
+    if (c1 - c <= kOwn * parts) {
+      for (long long k = c + part; k < c1; k += parts) w.chunk_first[k] = first_row(k * C - start, hdr);
+      c = c1;
+    }
+    for (unsigned long long many = __ballot(c < c1); many; many &= many - 1) {
+      const int l = __builtin_ctzll(many);
+      const long long c0 = lane_value(c, l), s0 = lane_value(start, l);
+      const int n = __builtin_amdgcn_readlane(int(c1 - c), l);
+      const int4 h = make_int4(__builtin_amdgcn_readlane(hdr.x, l), __builtin_amdgcn_readlane(hdr.y, l), 0,
+                               __builtin_amdgcn_readlane(hdr.w, l));
+      for (int k = part * kWave + lane; k < n; k += parts * kWave) w.chunk_first[c0 + k] = first_row((c0 + k) * C - s0, h);
+    }
+    __syncthreads();  // the shared arrays are rewritten by the next tile
+  }
+}
+
 // the nested lists; the first pass of the membership numbering
 __global__ void __launch_bounds__(kBlock) k_nested_members(DevView v, Work w, unsigned fill_blocks, long long n_mem,
                                                            MembershipScan mem, long long* ts_mem) {
@@ -1173,25 +1273,23 @@ __device__ __forceinline__ int gather_sources(const Work& w, int g, int cap, int
 // Wave path: one wavefront per row group
 // ---------------------------------------------------------------------------
 
-// a wave-uniform value loaded through the vector path, moved to a scalar register
-__device__ __forceinline__ long long uniform(long long x) {
-  const unsigned long long u = (unsigned long long)x;
-  return (long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(int(u >> 32)) << 32) |
-                     (unsigned)__builtin_amdgcn_readfirstlane(int(u & 0xffffffffu)));
-}
-
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ int wave_incl_scan(int x, int lane) {
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int y = __shfl_up(x, d, kWave);
-    if (lane >= d) x += y;
-  }
+// inclusive prefix sum over the wavefront, in six data-parallel-primitive adds (as
+// six permutes through LDS it is a chain of six LDS latencies): shifts by 1, 2, 4
+// and 8 inside each row of 16 lanes, then each row's last lane into the next row
+// (rows 1 and 3) and lane 31 into rows 2 and 3
+__device__ __forceinline__ int wave_incl_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
   return x;
 }
 
@@ -1239,8 +1337,8 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
     S.src_bs[lane] = int(b0);
     S.src_m0[lane] = m0;
   }
-  const int incl = wave_incl_scan(cnt, lane);
-  const int n_raw = __shfl(incl, kWave - 1, kWave);
+  const int incl = wave_incl_scan(cnt);
+  const int n_raw = __builtin_amdgcn_readlane(incl, kWave - 1);
   if (n_raw > kWR) return 1;
   if (lane < n_src) S.raw_base[lane] = incl - cnt;
   wave_sync();
@@ -1343,12 +1441,12 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
   for (int base = 0; base < n_dist; base += kWave) {
     const int t = base + lane;
     const int sz = t < n_dist ? S.cum[t] : 0;
-    const int inc = wave_incl_scan(sz, lane);
+    const int inc = wave_incl_scan(sz);
     if (t < n_dist) {
       S.cum[t] = carry + inc - sz;
       if (S.dstart[t] == gs_self) S.u_self = carry + inc - sz;
     }
-    carry += __shfl(inc, kWave - 1, kWave);
+    carry += __builtin_amdgcn_readlane(inc, kWave - 1);
   }
   if (lane == 0) {
     S.cum[n_dist] = carry;
@@ -1525,7 +1623,6 @@ constexpr int kBatchRows = 32;
 constexpr int kBatchSrc = kWS;       // sources of a batch's groups: those of any one group fit
 constexpr int kSrcBits = 5;
 constexpr int kBatchEntries = 1024;  // entries of a batch at most (bits of its row bitmap)
-constexpr int kMaxChunk = 4096;
 constexpr int kLargeRow = -0x7fffffff - 1;
 // a chunk meets at most kMaxChunk + 1 groups, so a record index fits beside the source
 static_assert(kBatchSrc <= 1 << kSrcBits && (kMaxChunk + 2) * kWC < 1 << (31 - kSrcBits), "FillRow::at_src");
@@ -1582,7 +1679,7 @@ __device__ __forceinline__ void fill_contrib(const double* __restrict__ lib, con
   l2 = ((c >> 5) & 1u) == dr ? l2v : 0.0;
 }
 
-// Streaming fill: the CSR is cut into chunks of w.chunk consecutive entries, which
+// Streaming fill: the CSR is cut into chunks (fill_chunk_of) of consecutive entries, which
 // the blocks take in rounds (FillRounds), a chunk for each wavefront.
 // A chunk is worked through in batches of up to kBatchRows rows: lane l prepares
 // row l of the batch (its start, from the group's segment, which is also its row
@@ -1610,15 +1707,16 @@ __global__ void __launch_bounds__(kFillBlock, kFillWavesPerSimd) k_fill_flat(Wor
   __shared__ double lib_lds[kLibInLds ? kFillLibLds : 1];
   const long long nnz = w.row_ptr[w.n_dofs];
   if (nnz > o.capacity) return;  // the host grows the buffers and runs the fill again
+  const long long chunk = uniform(fill_chunk(w, nnz));
+  const long long n_chunks = min((nnz + chunk - 1) / chunk, w.chunk_cap);
+  constexpr int kWaves = kFillBlock / kWave;
+  if (blockIdx.x * (long long)kWaves >= n_chunks) return;  // no chunk for this block
   if (kLibInLds) {
     const int n_lib = (L.nr + L.nr_v) * L.range_stride;
     for (int i = threadIdx.x; i < n_lib; i += blockDim.x) lib_lds[i] = w.lib[i];
   }
   const int lane = threadIdx.x % kWave;
   FillShared& S = shared[threadIdx.x / kWave];
-  const long long chunk = w.chunk;
-  const long long n_chunks = min((nnz + chunk - 1) / chunk, w.chunk_cap);
-  constexpr int kWaves = kFillBlock / kWave;
   const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   auto answer = [&](int k, int t) {  // one lane
     __hip_atomic_store(&rounds.ring[k % kRing], ((unsigned long long)unsigned(k + 1) << 32) | (gridDim.x + unsigned(t)),
@@ -1711,7 +1809,7 @@ __global__ void __launch_bounds__(kFillBlock, kFillWavesPerSimd) k_fill_flat(Wor
       }
       S.row[row].var[2 * k] = row_variant(spec_ahead, false, tab);
       S.row[row].var[2 * k + 1] = row_variant(spec_ahead, true, tab);
-      const int src_end = wave_incl_scan(lead && first ? n_src : 0, lane);  // sources up to and with the row's group
+      const int src_end = wave_incl_scan(lead && first ? n_src : 0);  // sources up to and with the row's group
       // the batch: entries [pos, limit), pieces of kWave from the multiple at or below pos
       const int at0 = pos & ~(kWave - 1);
       int limit = min(min(len, at0 + kBatchEntries), __builtin_amdgcn_readlane(end, kBatchRows - 1));
@@ -1853,15 +1951,10 @@ void launch_fill(int place, bool a_cc, bool b_cc, unsigned grid, hipStream_t st,
   }
 }
 
-// the library fits the fill's LDS copy of a placement (kPlaceGlobal always fits)
-bool place_fits(int place, long long lib_n) { return place == kPlaceGlobal || lib_n <= kFillLibLds; }
-
-// the placement an assembly uses: the tuned one, else the LDS copy when the
-// library fits it
-int fill_place(int tuned, long long lib_n) {
-  if (tuned >= 0 && place_fits(tuned, lib_n)) return tuned;
-  return place_fits(kPlaceLds, lib_n) ? kPlaceLds : kPlaceGlobal;
-}
+// The placement an assembly uses: the LDS copy when the library fits it (global
+// reads were slower on every Domain measured: 93 against 126 us on 25.7 M entries,
+// 382 against 517 us on 87 M).
+int fill_place(long long lib_n) { return lib_n <= kFillLibLds ? kPlaceLds : kPlaceGlobal; }
 
 // ---------------------------------------------------------------------------
 // Block path: one block per large row group
@@ -1891,7 +1984,7 @@ struct GroupShared {
 // *total receives the sum. Two barriers; every thread must call it.
 __device__ __forceinline__ int block_excl_scan(int x, int* wave_sum, int* total) {
   const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
-  const int incl = wave_incl_scan(x, lane);
+  const int incl = wave_incl_scan(x);
   if (lane == kWave - 1) wave_sum[wid] = incl;
   __syncthreads();
   int before = 0, all = 0;
@@ -2338,11 +2431,10 @@ struct GraphKey {
   bool run_large = true;
   int precision = -1;
   int chunk = 0;
-  int lib_lds = -1;
   bool operator==(const GraphKey& o) const {
     return domain == o.domain && basis == o.basis && ai == o.ai && bi == o.bi && nu == o.nu && nv == o.nv &&
            capacity == o.capacity && alloc_generation == o.alloc_generation && run_large == o.run_large &&
-           precision == o.precision && chunk == o.chunk && lib_lds == o.lib_lds;
+           precision == o.precision && chunk == o.chunk;
   }
 };
 
@@ -2367,11 +2459,6 @@ struct fem2d_device_domain {
   // whether any row group needs the block path: a property of the Domain,
   // learned by the first assembly (-1 unknown, 0 none, 1 some)
   mutable int large_state = -1;
-  // the streaming fill's chunk size and library placement (1 LDS, 0 global
-  // memory) per stored precision, chosen by timing the candidates on this
-  // Domain (chunk 0: not tuned yet)
-  mutable int tuned_chunk[kPrecisions] = {};
-  mutable int tuned_lds[kPrecisions] = {-1, -1, -1};
   // device arrays
   int* parent = nullptr;
   unsigned char* loc = nullptr;
@@ -2425,8 +2512,7 @@ struct fem2d_ctx {
   // global memory / in LDS
   int fill_grid[kPrecisions][2] = {};  // resident blocks of the fill per precision and FillPlace
   bool use_graphs = true;
-  bool autotune = true;  // time the fill's chunk sizes on a Domain's first assembly
-  int fill_chunk = 0;     // fill chunk size forced for every assembly (0: tuned or default)
+  int fill_chunk = 0;  // fill chunk size forced for every assembly (0: fill_chunk_of's)
   hipGraphExec_t graph_exec[1] = {nullptr};  // the last recorded assembly
   GraphKey graph_key;
   void* solver = nullptr;  // eigensolver handle, made by the first solve
@@ -2629,7 +2715,6 @@ struct Assembly {
   long long tiles_nested = 0, tiles_dof = 0, tiles_mem = 0, tiles_grp = 0;
   long long *ts_nested = nullptr, *ts_dof = nullptr, *ts_mem = nullptr, *ts_grp = nullptr;
   bool run_large = true;  // launch the block path (unless the Domain is known to need none)
-  int lib_lds = -1;       // the fill's FillPlace (-1: untuned, the LDS copy when it fits)
 };
 
 // Option and size checks after check_common; *nu, *nv receive the Gauss point counts.
@@ -2858,10 +2943,14 @@ int launch_prep(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, long long* st
   const unsigned large_grid = unsigned(std::max(1, ctx->n_cu * 2));
   if (a.run_large) k_count_large<<<large_grid, kBlock, sizeof(GroupShared), st>>>(v, w);
   HIP_TRY_AT(hipGetLastError(), "after the describe kernels");
-  // CSR layout and the status block
-  const GroupScan gs{w, a.n_grp_items, status};
-  k_scan_reduce<<<scan_grid(a.tiles_grp), kBlock, 0, st>>>(a.n_grp_items, gs, a.ts_grp);
-  k_scan_apply<<<scan_grid(a.tiles_grp), kBlock, 0, st>>>(a.n_grp_items, gs, a.ts_grp);
+  // CSR layout and the status block; up to kLayoutTiles tiles of groups the second
+  // pass sums the tiles itself (a launch less)
+  constexpr long long kLayoutTiles = 8;
+  const bool two_pass = a.tiles_grp > kLayoutTiles;
+  const int parts = two_pass ? 1 : 8;
+  if (two_pass) k_scan_reduce<<<scan_grid(a.tiles_grp), kBlock, 0, st>>>(a.n_grp_items, GroupScan{w}, a.ts_grp);
+  k_layout<<<scan_grid(a.tiles_grp) * unsigned(parts), kBlock, 0, st>>>(w, a.n_grp_items,
+                                                                        two_pass ? a.ts_grp : nullptr, parts, status);
   HIP_TRY_AT(hipGetLastError(), "after the CSR layout scan");
   if (fine_events) HIP_TRY(hipEventRecord(ctx->ev[2], st));
   return FEM2D_OK;
@@ -2871,7 +2960,7 @@ int launch_prep(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, long long* st
 // buffers it writes nothing)
 int launch_stream_fill(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, const FillOut& o) {
   const int pi = o.precision;
-  const int place = fill_place(a.lib_lds, a.lib_n);
+  const int place = fill_place(a.lib_n);
   launch_fill(place, o.a_is_cc != 0, o.b_is_cc != 0, unsigned(ctx->fill_grid[pi][place]), st, a.w, a.L, o);
   HIP_TRY_AT(hipGetLastError(), "after the fill kernel");
   return FEM2D_OK;
@@ -2911,22 +3000,15 @@ FillOut make_fill_out(int precision, int ai, int bi, long long capacity, int* co
   return o;
 }
 
-// chunk sizes the fill's autotuning times on a Domain's first assembly, each
-// placement and size timed kTuneReps times (the fastest launch counts)
-constexpr int kChunkCandidates[] = {256, 512, 768};
-constexpr int kTuneReps = 5;
+// chunk_max per stored precision (fill_chunk_of has the measurements)
+constexpr int chunk_max_of(int precision) { return precision == FEM2D_PRECISION_FP32 ? 768 : 512; }
 
-// FEM2D_TUNE_VERBOSE=1 prints every tuning trial's time to stderr
-bool tune_verbose() {
-  static const bool on = [] {
-    const char* e = std::getenv("FEM2D_TUNE_VERBOSE");
-    return e != nullptr && e[0] != '\0' && e[0] != '0';
-  }();
-  return on;
+// The chunk size and launch of an assembly's fill; the caller sets chunk_cap.
+void set_chunk(const fem2d_ctx* ctx, Assembly& a, int precision) {
+  a.w.chunk = ctx->fill_chunk;
+  a.w.chunk_max = chunk_max_of(precision);
+  a.w.fill_waves = ctx->fill_grid[precision][fill_place(a.lib_n)] * (kFillBlock / kWave);
 }
-
-// w.chunk for a chunk size (0: the default)
-void set_chunk(Work& w, int chunk) { w.chunk = chunk > 0 ? chunk : kFillChunk; }
 
 // Host metadata of a device Domain that depends on the Elem tree only: the
 // sub-ranges of the Gram library (the position of each Elem inside each of its
@@ -3118,7 +3200,7 @@ int fem2d_ctx_set_autotune(fem2d_ctx* ctx, int enable) {
     set_error("null argument", 0);
     return FEM2D_ERR_INVALID_ARG;
   }
-  ctx->autotune = enable != 0;
+  (void)enable;  // the fill's chunk size and library placement follow from sizes alone
   return FEM2D_OK;
 }
 
@@ -3127,7 +3209,7 @@ int fem2d_ctx_set_fill_chunk(fem2d_ctx* ctx, int chunk) {
     set_error("null argument", 0);
     return FEM2D_ERR_INVALID_ARG;
   }
-  if (chunk != 0 && (chunk < kWave || chunk > 4096 || (chunk & (chunk - 1)) != 0)) {
+  if (chunk != 0 && (chunk < kWave || chunk > kMaxChunk || (chunk & (chunk - 1)) != 0)) {
     set_error("fill chunk: 0, or a power of two from 64 to 4096", 0);
     return FEM2D_ERR_INVALID_ARG;
   }
@@ -3301,8 +3383,8 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
                      [&](int k, size_t count, auto** ptr) { return slot(ctx, k, count, ptr); }, a);
   if (!rc) rc = slot(ctx, kRowPtrSlot, size_t(nd + 1), &a.w.row_ptr);
   if (rc) return rc;
-  a.lib_lds = dd->tuned_lds[precision];
   Work& w = a.w;
+  set_chunk(ctx, a, precision);
   const bool run_large = a.run_large;
   hipStream_t st = ctx->stream;
   ensure_glq(ctx, nu, nv);
@@ -3346,14 +3428,13 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
       return rc;
     const FillOut o = make_fill_out(precision, ai, bi, ctx->out_capacity, static_cast<int*>(ctx->out_col.p),
                                     ctx->out_a.p, ctx->out_b.p, static_cast<unsigned*>(ctx->out_r.p));
-    set_chunk(w, ctx->fill_chunk ? ctx->fill_chunk : dd->tuned_chunk[precision]);
-    w.chunk_cap = o.capacity / w.chunk + 1;
+    w.chunk_cap = w.chunk ? o.capacity / w.chunk + 1 : fill_chunk_cap(o.capacity, w.fill_waves, w.chunk_max);
     if ((rc = slot(ctx, kChunkSlot, size_t(w.chunk_cap), &w.chunk_first))) return rc;
     const bool fill = o.capacity > 0;
     const bool tail = fill && run_large;  // part (c) has work
     if (ctx->use_graphs) {
       const GraphKey key{dd->serial, basis,     ai,       bi, nu, nv, o.capacity, g_alloc_generation.load(),
-                         run_large,  precision, w.chunk, a.lib_lds};
+                         run_large,  precision, w.chunk};
       if (!ctx->graph_exec[0] || !(key == ctx->graph_key)) {
         ctx->graph_key = GraphKey{};
         if ((rc = record(0, [&] {
@@ -3418,50 +3499,8 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
     return fem2d_assemble_device(ctx, dd, basis, ai, bi, glq_u, glq_v, precision, out);
   }
   dd->large_state = n_large > 0 ? 1 : 0;
-  a.run_large = n_large > 0;  // the tuning trials below skip the block path's count when it has no group
-  ctx->timing.fill_chunk = w.chunk;
-  ctx->timing.fill_lib_lds = fill_place(a.lib_lds, a.lib_n);
-  if (ctx->autotune && !ctx->fill_chunk && dd->tuned_chunk[precision] == 0) {
-    // the first assembly of this Domain in this precision: time the streaming
-    // fill at each candidate chunk size and library placement (best of
-    // kTuneReps launches each, after the layout scan for that size), keep the fastest,
-    // and assemble again with it
-    int best = w.chunk, best_lds = -1;
-    float best_ms = HUGE_VALF;
-    const FillOut o = make_fill_out(precision, ai, bi, ctx->out_capacity, static_cast<int*>(ctx->out_col.p),
-                                    ctx->out_a.p, ctx->out_b.p, static_cast<unsigned*>(ctx->out_r.p));
-    // the repetitions are the outer loop, so that a drift of the GPU's clocks
-    // over the trials favours no candidate
-    for (int rep = 0; rep < kTuneReps; ++rep)
-      for (int place : {kPlaceLds, kPlaceGlobal}) {
-        if (!place_fits(place, a.lib_n)) continue;
-        a.lib_lds = place;
-        for (int c : kChunkCandidates) {
-          set_chunk(w, c);
-          w.chunk_cap = o.capacity / w.chunk + 1;
-          if ((rc = slot(ctx, kChunkSlot, size_t(w.chunk_cap), &w.chunk_first))) return rc;
-          if ((rc = launch_prep(ctx, st, a, ctx->d_status, false))) return rc;
-          HIP_TRY(hipEventRecord(ctx->ev[6], st));
-          if ((rc = launch_stream_fill(ctx, st, a, o))) return rc;
-          HIP_TRY(hipEventRecord(ctx->ev[7], st));
-          HIP_TRY(hipStreamSynchronize(st));
-          float ms = 0.0f;
-          HIP_TRY(hipEventElapsedTime(&ms, ctx->ev[6], ctx->ev[7]));
-          if (ctx->h_status[1]) return err_to_status(ctx->h_status[1]);
-          if (tune_verbose())
-            std::fprintf(stderr, "[fem2d tune] precision %d placement %d chunk %d: %.4f ms\n", precision, place, c,
-                         double(ms));
-          if (ms < best_ms) {
-            best_ms = ms;
-            best = c;
-            best_lds = place;
-          }
-        }
-      }
-    dd->tuned_chunk[precision] = best;
-    dd->tuned_lds[precision] = best_lds;
-    return fem2d_assemble_device(ctx, dd, basis, ai, bi, glq_u, glq_v, precision, out);
-  }
+  ctx->timing.fill_chunk = w.chunk ? w.chunk : fill_chunk_of(nnz, w.chunk_cap, w.fill_waves, w.chunk_max);
+  ctx->timing.fill_lib_lds = fill_place(a.lib_n);
 
   out->n = nd;
   out->nnz = nnz;
@@ -3517,11 +3556,16 @@ int fem2d_assemble_device_noalloc(fem2d_ctx* ctx, const fem2d_device_domain* dd,
                      },
                      a);
   if (rc) return rc;
-  a.lib_lds = dd->tuned_lds[precision];
   Work& w = a.w;
   w.row_ptr = row_ptr;
-  set_chunk(w, ctx->fill_chunk ? ctx->fill_chunk : dd->tuned_chunk[precision]);
-  w.chunk_cap = capacity / w.chunk + 1;
+  set_chunk(ctx, a, precision);
+  // the table of first rows comes last and takes what is left where that is less
+  // than it would like (larger chunks then)
+  const size_t at = (used + 255) & ~size_t(255);
+  const long long left = at < kScratchBytes ? (long long)((kScratchBytes - at) / sizeof(int)) : 0;
+  w.chunk_cap = w.chunk ? capacity / w.chunk + 1
+                        : std::max<long long>(std::min<long long>(fill_chunk_cap(capacity, w.fill_waves, w.chunk_max), left),
+                                   capacity / kMaxChunk + 1);
   w.chunk_first = static_cast<int*>(carve(size_t(w.chunk_cap) * sizeof(int)));
   if (used > kScratchBytes) {
     set_error("the assembly of this Domain needs " + std::to_string(used) + " bytes of work memory; the " +

@@ -94,13 +94,13 @@ class Context:
         check(self._lib.fem2d_ctx_set_graphs(self._h, 1 if enable else 0))
 
     def set_autotune(self, enable: bool) -> None:
-        """Time the entry fill's chunk sizes on each Domain's first assembly and keep the fastest
-        (default), or keep the default chunk size."""
+        """Accepted for callers of earlier versions: the entry fill's chunk size follows from the
+        GEP's size and nothing is timed."""
         check(self._lib.fem2d_ctx_set_autotune(self._h, 1 if enable else 0))
 
     def set_fill_chunk(self, chunk: int) -> None:
         """Forces the fill's chunk size (a power of two from 64 to 4096 CSR entries) for later
-        assemblies, with no tuning; 0 returns to the tuned or default size."""
+        assemblies; 0 returns to the size that follows from the GEP's."""
         check(self._lib.fem2d_ctx_set_fill_chunk(self._h, int(chunk)))
 
     def last_eigen_stats(self) -> dict:

@@ -153,16 +153,13 @@ int fem2d_ctx_synchronize(fem2d_ctx* ctx);
  * replayed (default 1) or launched kernel by kernel (0). Results are the same;
  * graphs remove the per-kernel launch gaps of the ~20-kernel pipeline. */
 int fem2d_ctx_set_graphs(fem2d_ctx* ctx, int enable);
-/* Whether the first assembly of a Domain in a precision times the entry fill at
- * each candidate chunk size (128, 256, 512, 1024 CSR entries per work item) and
- * library placement (an LDS copy per block when it fits, or global memory) and
- * keeps the fastest for later assemblies of that Domain (default 1). The tuned
- * shape changes timing only, never results. */
+/* Accepted for callers of earlier versions, which timed the entry fill's shapes on a
+ * Domain's first assembly: its chunk size and library placement now follow from
+ * the sizes alone, and this call changes nothing. */
 int fem2d_ctx_set_autotune(fem2d_ctx* ctx, int enable);
 /* Forces the streaming fill's chunk size (CSR entries per wavefront work item,
- * a power of two from 64 to 4096) for every later assembly on the context, with
- * no tuning while set; 0 returns to the tuned or default size. Results do not
- * depend on it. */
+ * a power of two from 64 to 4096) for every later assembly on the context; 0
+ * returns to the size that follows from the GEP's. Results do not depend on it. */
 int fem2d_ctx_set_fill_chunk(fem2d_ctx* ctx, int chunk);
 
 /* Replaces galerkin_sample_gep_hcurl (galerkin.rs:33-187).
@@ -389,9 +386,8 @@ typedef struct fem2d_timing {
   double fill_kernel_ms;  /* the wave-per-group entry-writing kernel alone */
   int64_t nnz;
   int64_t n_large;    /* row groups assembled one block per group (large column sets) */
-  int64_t fill_chunk; /* CSR entries per work item of the entry fill (default, tuned or forced) */
-  int64_t fill_lib_lds; /* where the entry fill read the Gram library: 0 global memory, 1 an LDS copy,
-                           2 an LDS copy in 512-thread blocks (default or tuned) */
+  int64_t fill_chunk; /* CSR entries per work item of the entry fill */
+  int64_t fill_lib_lds; /* where the entry fill read the Gram library: 0 global memory, 1 an LDS copy */
 } fem2d_timing;
 int fem2d_ctx_last_timing(fem2d_ctx* ctx, fem2d_timing* out);
 
