@@ -2300,116 +2300,132 @@ __global__ void __launch_bounds__(kBlock) k_fill_large(DevView v, Work w, LibSha
 // Field evaluation: UniformFieldSpace::xy_fields (fields.rs:63-127)
 // ---------------------------------------------------------------------------
 
-// Halves [lo, hi] per axis down a chain of HRefLocs (h_refinement.rs:247-279),
-// locs[from - 1] first (the step nearest the top), locs[to] last.
-__device__ __forceinline__ void fold_range(const unsigned char* locs, int from, int to, double& u0, double& u1,
-                                           double& v0, double& v1) {
-  u0 = -1.0; u1 = 1.0; v0 = -1.0; v1 = 1.0;
-  for (int t = from - 1; t >= to; --t) {
-    const double mu = (u0 + u1) / 2.0, mv = (v0 + v1) / 2.0;
-    const int l = locs[t];
-    const bool split_u = l <= FEM2D_LOC_E;
-    const bool split_v = l <= FEM2D_LOC_NE || l >= FEM2D_LOC_S;
-    const bool hi_u = l == FEM2D_LOC_SE || l == FEM2D_LOC_NE || l == FEM2D_LOC_E;
-    const bool hi_v = l == FEM2D_LOC_NW || l == FEM2D_LOC_NE || l == FEM2D_LOC_N;
-    if (split_u) {
-      if (hi_u) u0 = mu; else u1 = mu;
-    }
-    if (split_v) {
-      if (hi_v) v0 = mv; else v1 = mv;
-    }
-  }
+// A leaf's grid, one wavefront per tile of up to kFieldTile x kFieldTile points:
+// the sum over the leaf and its ancestors (leaf first, as Mesh::ancestor_elems
+// lists them) of the fields of each one's basis specs (basis.rs:225-233) at the
+// points mapped into its parametric space (defined_over with the leaf as
+// descendant, basis.rs:365-423). On one Elem the fields are
+//   x: ju0 sum_ij U_ij N_i(x) T_j(y),  y: jv1 sum_ij V_ij T_i(x) N_j(y)
+// with U and V the DoF values of its U and V specs, so the sums factor: the
+// shapes of every order at the tile's d + d coordinates once, the sums over j for
+// each coordinate y, then the sums over i for each point. With p orders that is
+// p p d + p d d products a direction instead of 2 p p d d, and 2 p d shape
+// evaluations instead of 4 p p d d (one point a thread, every shape evaluated
+// for every spec and point: 251 us for 6 350 leaves of 12 x 12 points at order 6; now 30 us).
+// The Jacobian's zero off-diagonal terms (space.rs:138-147) are added as the
+// reference adds them: -0 times the other direction's sum, which matters where a DoF
+// value is not finite.
+constexpr int kFieldTile = 16;
+constexpr int kFieldPoints = kFieldTile * kFieldTile / kWave;  // points a lane (those past the grid are dropped)
+
+constexpr int kFieldWavesPerSimd = 6;
+
+// LDS of the field kernel: coefficients of both directions, N and T on both axes,
+// the sums over j of both directions
+size_t field_lds_bytes(int p1) {
+  return size_t(2 * p1 * p1 + 6 * p1 * kFieldTile) * sizeof(double);
 }
 
-// One thread per grid point (leaf k, u point m, v point n) of every leaf:
-// the sum over the leaf and its ancestors (leaf first, as
-// Mesh::ancestor_elems lists them), over each one's basis specs in list
-// order, of f_u or f_v (basis.rs:225-233) at the point mapped into that
-// Elem's parametric space (defined_over with the leaf as descendant,
-// basis.rs:365-423), times the spec's DoF value. Every product is formed in
-// the reference's order: (jac_inv row * shape) * shape, then * solution, with
-// jac_inv = [[b, -0], [-0, a]] / (a b) (space.rs:138-147).
 template <int kBasis>
-__global__ void __launch_bounds__(kBlock) k_xy_fields(DevView v, const int* __restrict__ leaves, long long n_leaves,
-                                                      int d, const double* __restrict__ pts,
-                                                      const double* __restrict__ sol, double* __restrict__ fx,
-                                                      double* __restrict__ fy, int* __restrict__ err) {
-  const long long per_leaf = (long long)d * d;
-  const long long total = n_leaves * per_leaf;
-  for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
-       idx += (long long)gridDim.x * blockDim.x) {
-    const int leaf = leaves[idx / per_leaf];
-    const int m = int((idx / d) % d), n = int(idx % d);
-    unsigned char locs[kMaxDepth];
-    int depth = 0;
-    bool ok = true;
-    for (int x = leaf; v.parent[x] >= 0;) {
-      const int p = v.parent[x];
-      if (p >= v.n_elems || p == x || depth >= kMaxDepth || v.loc[x] > FEM2D_LOC_N) {
-        ok = false;
-        break;
-      }
-      locs[depth++] = v.loc[x];
-      x = p;
-    }
-    double sx = 0.0, sy = 0.0;
-    if (!ok) {
-      set_err(err, kErrView);
-      fx[idx] = sx;
-      fy[idx] = sy;
-      continue;
-    }
-    int A = leaf;
-    for (int t = 0; t <= depth; ++t) {
-      // the Elem t steps above the leaf: its parametric range and Jacobian
-      // (element.rs:33-50) ...
-      double u0, u1, v0, v1;
-      fold_range(locs, depth, t, u0, u1, v0, v1);
-      const double* bx = v.box + 4 * A;
-      const double a = (map_range(u1, -1.0, 1.0, bx[0], bx[2]) - map_range(u0, -1.0, 1.0, bx[0], bx[2])) / 2.0;
-      const double b = (map_range(v1, -1.0, 1.0, bx[1], bx[3]) - map_range(v0, -1.0, 1.0, bx[1], bx[3])) / 2.0;
-      const double det = a * b - 0.0 * 0.0;
-      const double ju0 = b / det, jz = (-1.0 * 0.0) / det, jv1 = a / det;
-      // ... and the leaf's grid point in it (glq.rs:238-249 over the leaf's
-      // range relative to this Elem; the leaf itself takes the points as given)
-      double x = pts[m], y = pts[n];
-      if (t > 0) {
-        double r0, r1, q0, q1;
-        fold_range(locs, t, 0, r0, r1, q0, q1);
-        x = x * ((r1 - r0) / 2.0) + (r1 + r0) / 2.0;
-        y = y * ((q1 - q0) / 2.0) + (q1 + q0) / 2.0;
-      }
-      for (long long k = v.bs_off[A]; k < v.bs_off[A + 1]; ++k) {
-        const int dof = v.bs_dof[k];
-        if (dof < 0 || dof >= v.n_dofs) {
-          set_err(err, kErrView);
-          continue;
-        }
-        const int dir = v.bs_dir[k], i = v.bs_i[k], j = v.bs_j[k];
-        const double s = sol[dof];
-        double Nu, Ndu, Tu, Tdu, Nv, Ndv, Tv, Tdv;
-        if (kBasis == FEM2D_BASIS_KOL) {
-          kol(i, x, Nu, Ndu, Tu, Tdu);
-          kol(j, y, Nv, Ndv, Tv, Tdv);
-        } else {
-          hier_poly(i, x, Nu, Ndu, Tu, Tdu);
-          hier_poly(j, y, Nv, Ndv, Tv, Tdv);
-        }
-        if (dir == 0) {  // f_u = jac_inv.u * N_i(x) * T_j(y)
-          sx += ((ju0 * Nu) * Tv) * s;
-          sy += ((jz * Nu) * Tv) * s;
-        } else if (dir == 1) {  // f_v = jac_inv.v * T_i(x) * N_j(y)
-          sx += ((jz * Tu) * Nv) * s;
-          sy += ((jv1 * Tu) * Nv) * s;
-        } else {  // any other direction contributes the zero vector times the DoF value
-          sx += 0.0 * s;
-          sy += 0.0 * s;
+__global__ void __launch_bounds__(kWave, kFieldWavesPerSimd) k_xy_fields(DevView v, const ElemGeo* __restrict__ geo,
+                                                     const int4* __restrict__ dyad, const unsigned* __restrict__ bs_pack,
+                                                     const int* __restrict__ leaves, long long n_leaves, int d,
+                                                     double step, const double* __restrict__ sol,
+                                                     double* __restrict__ fx, double* __restrict__ fy) {
+  extern __shared__ double field_lds[];
+  constexpr int kRows = kWave / kFieldTile;
+  const int p1 = v.p1, lane = threadIdx.x;
+  const int k = lane % kFieldTile, q = lane / kFieldTile;  // point m = q + kRows h, n = k of the tile
+  double* coef = field_lds;                     // [2][p1][p1] by direction, i, j
+  double* shape = coef + 2 * p1 * p1;           // [axis][N, T][p1][kFieldTile]
+  double* part = shape + 4 * p1 * kFieldTile;   // [2][p1][kFieldTile] sums over j
+  const int tiles = (d + kFieldTile - 1) / kFieldTile;
+  const long long items = n_leaves * tiles * tiles;
+  for (long long item = blockIdx.x; item < items; item += gridDim.x) {
+    const int leaf = ld_const(leaves, item / (tiles * tiles));
+    const int tile = int(item % (tiles * tiles));
+    const int m0 = tile / tiles * kFieldTile, n0 = tile % tiles * kFieldTile;
+    const int dm = min(kFieldTile, d - m0), dn = min(kFieldTile, d - n0);
+    const int4 at = dyad[leaf];
+    double sx[kFieldPoints] = {}, sy[kFieldPoints] = {};
+    for (int A = leaf; A >= 0; A = ld_const(v.parent, A)) {
+      const int4 up = dyad[A];
+      // the leaf's range in A on each axis (exact: powers of two)
+      double su, cu, sv, cv;
+      range_of(range_key(at.x - up.x, at.y - (up.y << (at.x - up.x))), su, cu);
+      range_of(range_key(at.z - up.z, at.w - (up.w << (at.z - up.z))), sv, cv);
+      const bool own = A == leaf;  // the leaf takes the points as given
+      const long long t0 = v.bs_off[A], t1 = v.bs_off[A + 1];
+      if (t0 == t1) continue;  // adds nothing, not even at the NaN point of a 1 x 1 grid
+      // the first two specs a lane load while the tables are filled
+      unsigned pk[2] = {0u, 0u};
+      double val[2] = {0.0, 0.0};
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const long long t = t0 + h * kWave + lane;
+        if (t < t1) {
+          pk[h] = bs_pack[t];
+          val[h] = sol[v.bs_dof[t]];
         }
       }
-      A = v.parent[A];
+      for (int i = lane; i < 2 * p1 * p1; i += kWave) coef[i] = 0.0;
+      // rows r of kFieldTile values: axis 0 (r < p1) or 1 and an order
+      for (int r = q; r < 2 * p1; r += kRows) {
+        const int axis = r >= p1 ? 1 : 0, n = r - axis * p1;
+        double x = double((axis ? n0 : m0) + k) * step + -1.0;
+        if (!own) x = axis ? x * sv + cv : x * su + cu;
+        double N, Nd, T, Td;
+        if (kBasis == FEM2D_BASIS_KOL) kol(n, x, N, Nd, T, Td);
+        else hier_poly(n, x, N, Nd, T, Td);
+        shape[((axis * 2 + 0) * p1 + n) * kFieldTile + k] = N;
+        shape[((axis * 2 + 1) * p1 + n) * kFieldTile + k] = T;
+      }
+      wave_sync();
+      auto add = [&](unsigned spec, double value) {
+        unsafeAtomicAdd(&coef[(spec_dir(spec) * p1 + spec_i(spec)) * p1 + spec_j(spec)], value);
+      };
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (t0 + h * kWave + lane < t1) add(pk[h], val[h]);
+      for (long long t = t0 + 2 * kWave + lane; t < t1; t += kWave) add(bs_pack[t], sol[v.bs_dof[t]]);
+      wave_sync();
+      for (int r = q; r < 2 * p1; r += kRows) {  // direction 0 (r < p1) or 1 and i
+        const double* c = coef + r * p1;
+        const double* y = shape + (r < p1 ? 3 : 2) * p1 * kFieldTile + k;  // T_j or N_j of y
+        double sum = 0.0;
+#pragma unroll 4
+        for (int j = 0; j < p1; ++j) sum += c[j] * y[j * kFieldTile];
+        part[r * kFieldTile + k] = sum;
+      }
+      wave_sync();
+      const ElemGeo g = geo[A];
+      const double jz = -0.0;
+      double u[kFieldPoints] = {}, w[kFieldPoints] = {};
+#pragma unroll 2
+      for (int a = 0; a < p1; ++a) {
+        const double pu = part[a * kFieldTile + k], pw = part[(p1 + a) * kFieldTile + k];
+        const double *xu = shape + a * kFieldTile + q, *xw = xu + p1 * kFieldTile;
+#pragma unroll
+        for (int h = 0; h < kFieldPoints; ++h) {
+          u[h] += xu[h * kRows] * pu;
+          w[h] += xw[h * kRows] * pw;
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < kFieldPoints; ++h) {
+        sx[h] += g.ju0 * u[h] + jz * w[h];
+        sy[h] += jz * u[h] + g.jv1 * w[h];
+      }
+      wave_sync();  // the tables are rewritten for the next Elem
     }
-    fx[idx] = sx;
-    fy[idx] = sy;
+#pragma unroll
+    for (int h = 0; h < kFieldPoints; ++h) {
+      const int m = h * kRows + q;
+      if (m >= dm || k >= dn) continue;
+      const long long o = (item / (tiles * tiles) * d + m0 + m) * d + n0 + k;
+      fx[o] = sx[h];
+      fy[o] = sy[h];
+    }
   }
 }
 
@@ -2496,7 +2512,6 @@ struct fem2d_ctx {
   std::vector<DevBuf> bufs;  // grow-only work buffers, by slot
   DevBuf out_col, out_a, out_b;
   DevBuf out_r;  // FP32R residuals (grown on the first FP32R assembly that needs them)
-  DevBuf field_scratch;  // grid points and status word of the field evaluation
   long long out_capacity = 0;
   long long* h_status = nullptr;  // mapped pinned status block: nnz, err, n_large, n_groups
   void* h_stage = nullptr;        // pinned upload staging of the device Domain builder (grow-only)
@@ -3159,7 +3174,7 @@ void fem2d_ctx_destroy(fem2d_ctx* ctx) {
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   for (auto& b : ctx->bufs)
     if (b.p) (void)hipFree(b.p);
-  for (DevBuf* b : {&ctx->out_col, &ctx->out_a, &ctx->out_b, &ctx->out_r, &ctx->field_scratch})
+  for (DevBuf* b : {&ctx->out_col, &ctx->out_a, &ctx->out_b, &ctx->out_r})
     if (b->p) (void)hipFree(b->p);
   for (auto& g : ctx->graph_exec)
     if (g) (void)hipGraphExecDestroy(g);
@@ -3691,54 +3706,21 @@ int fem2d_device_xy_fields(fem2d_ctx* ctx, const fem2d_device_domain* dd, int ba
     return FEM2D_ERR_INVALID_ARG;
   }
   HIP_TRY(hipSetDevice(ctx->device));
-  // uniform_range(-1.0, 1.0, d) (fields.rs:402-405), followed by a zeroed
-  // status word, staged in one copy to the context's scratch buffer
-  std::vector<double> pts(static_cast<size_t>(d) + 1, 0.0);
+  // uniform_range(-1.0, 1.0, d) (fields.rs:402-405): point i is i step - 1
   const double step = (1.0 - -1.0) / double(d - 1);
-  for (int i = 0; i < d; ++i) pts[size_t(i)] = double(i) * step + -1.0;
-  int rc = ensure(ctx->field_scratch, pts.size() * sizeof(double));
-  double* d_pts = static_cast<double*>(ctx->field_scratch.p);
-  int* d_err = reinterpret_cast<int*>(d_pts + d);
-  if (!rc) {
-    hipError_t e = hipMemcpyAsync(d_pts, pts.data(), pts.size() * sizeof(double), hipMemcpyHostToDevice,
-                                  ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // pts is read before any return below
-    if (e != hipSuccess) rc = hip_fail(e, "field grid upload");
-  }
-  if (!rc) {
-    DevView v{};
-    v.n_elems = dd->n_elems;
-    v.n_dofs = dd->n_dofs;
-    v.n_bs = dd->n_bs;
-    v.parent = dd->parent;
-    v.loc = dd->loc;
-    v.box = dd->box;
-    v.mat = dd->mat;
-    v.bs_off = dd->bs_off;
-    v.bs_dir = dd->bs_dir;
-    v.bs_i = dd->bs_i;
-    v.bs_j = dd->bs_j;
-    v.bs_dof = dd->bs_dof;
-    v.dof_bs = dd->dof_bs;
-    const unsigned grid =
-        unsigned(std::min<long long>((total + kBlock - 1) / kBlock, std::max(1, ctx->n_cu) * 16LL));
-    if (basis == FEM2D_BASIS_KOL)
-      k_xy_fields<FEM2D_BASIS_KOL><<<grid, kBlock, 0, ctx->stream>>>(v, dd->leaves, dd->n_leaves, d, d_pts, solution,
-                                                                    out_x, out_y, d_err);
-    else
-      k_xy_fields<FEM2D_BASIS_HIERPOLY><<<grid, kBlock, 0, ctx->stream>>>(v, dd->leaves, dd->n_leaves, d, d_pts,
-                                                                         solution, out_x, out_y, d_err);
-    hipError_t e = hipGetLastError();
-    int h_err = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&h_err, d_err, sizeof(int), hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) rc = hip_fail(e, "field evaluation");
-    else if (h_err) {
-      set_error("domain view violates the Domain invariants (parent chain, location or DoF id)", 0);
-      rc = FEM2D_ERR_INVALID_VIEW;
-    }
-  }
-  return rc;
+  const DevView v = dev_view(dd);
+  const long long tiles = (d + kFieldTile - 1) / kFieldTile;
+  const unsigned grid = unsigned(std::min<long long>(dd->n_leaves * tiles * tiles, std::max(1, ctx->n_cu) * 128LL));
+  const size_t lds = field_lds_bytes(v.p1);
+  if (basis == FEM2D_BASIS_KOL)
+    k_xy_fields<FEM2D_BASIS_KOL><<<grid, kWave, lds, ctx->stream>>>(v, dd->geo, dd->dyad, dd->bs_pack, dd->leaves,
+                                                                   dd->n_leaves, d, step, solution, out_x, out_y);
+  else
+    k_xy_fields<FEM2D_BASIS_HIERPOLY><<<grid, kWave, lds, ctx->stream>>>(
+        v, dd->geo, dd->dyad, dd->bs_pack, dd->leaves, dd->n_leaves, d, step, solution, out_x, out_y);
+  HIP_TRY_AT(hipGetLastError(), "after the field kernel");
+  HIP_TRY_AT(hipStreamSynchronize(ctx->stream), "after the field kernel");
+  return FEM2D_OK;
 }
 
 int fem2d_xy_fields(fem2d_ctx* ctx, const fem2d_domain_view* view, int basis, int density_u, int density_v,
