@@ -112,8 +112,7 @@ constexpr int kMaxChunk = 4096;  // CSR entries per work item (chunk) of the fil
 // placements of the fill's Gram library: global memory, or an LDS copy
 enum FillPlace { kPlaceGlobal = 0, kPlaceLds = 1 };
 constexpr int kFillWavesPerSimd = 4;
-// latency-bound kernels: at most 64 VGPRs, so that 8 wavefronts per SIMD are resident
-constexpr int kLatencyWavesPerSimd = 8;
+constexpr int kDescribeWavesPerSimd = 6;
 constexpr int kMaxDepth = 24;      // h-refinement depth below a base Elem
 constexpr int kMaxRanges = 16383;  // distinct relative sub-ranges per axis (14-bit ids in the block path)
 // spec_pos bits: a spec's index in its Elem's list, and flags
@@ -1293,26 +1292,37 @@ __device__ __forceinline__ int wave_incl_scan(int x) {
   return x;
 }
 
-// Per-wave LDS of the candidate-set build (both wave kernels)
+// Per-wave LDS of the candidate-set build by a whole wavefront
 struct WaveShared {
   int src_x[kWS];
   int src_info[kWS];  // k | rel << 1 | ru << 3 | rv << 17
   int src_bs[kWS];    // first basis spec of each source (bs_offsets)
   int src_m0[kWS];    // first membership of each source
   int raw_base[kWS];  // first raw candidate of each source
-  union {
-    struct {
-      unsigned long long key[kWR];  // row group << 20 | raw index
-      int raw_meta[kWR];            // source | bs offset << 8
-    } sort;
-    uint2 row_pk[kWRows];  // fill: packed specs of the group's rows on its first / second Elem
-  } u;
+  unsigned long long key[kWR];  // row group << 20 | raw index
+  int raw_meta[kWR];            // source | bs offset << 8
   int dstart[kWD];
   int cum[kWD + 1];
   int dmeta0[kWD];  // source | bs offset << 8 of the first contribution to a candidate group
   int dmeta1[kWD];  // the same for the second contribution, -1 if none
   int n_src, n_dist, total, u_self;
 };
+
+// The record of a source in the fill: per column direction the CurlCurl prefactors
+// by row direction (the p side of the pair is the column's where the source is an
+// ancestor), the L2Inner prefactor and the library bases
+__device__ __forceinline__ void write_source(const Work& w, double* out, const double* cA, const double* cB, int ru,
+                                             int rv, bool anc) {
+  const int2 base = make_int2(8 * (ru * w.lib_range_stride), 8 * ((w.lib_nr + rv) * w.lib_range_stride + w.lib_tab));
+  out[0] = cA[0];
+  out[1] = anc ? cA[1] : cA[2];
+  out[4] = anc ? cA[2] : cA[1];
+  out[5] = cA[3];
+  for (int d = 0; d < 2; ++d) {
+    out[4 * d + 2] = cB[d];
+    *reinterpret_cast<int2*>(out + 4 * d + 3) = base;
+  }
+}
 
 // Builds row group g's candidate set in this wave's LDS slice. Returns 0 when
 // built and inside the wave path's limits, 1 when the group needs the block
@@ -1351,8 +1361,8 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
       if (S.raw_base[mid] <= r) a = mid; else b = mid;
     }
     const int m = S.src_m0[a] + (r - S.raw_base[a]);
-    S.u.sort.key[r] = ((unsigned long long)(unsigned)w.mem_group[m] << 20) | (unsigned long long)r;
-    S.u.sort.raw_meta[r] = a | (w.mem_bsoff[m] << 8);
+    S.key[r] = ((unsigned long long)(unsigned)w.mem_group[m] << 20) | (unsigned long long)r;
+    S.raw_meta[r] = a | (w.mem_bsoff[m] << 8);
   }
   if (lane < n_src) {
     if (coef) {
@@ -1364,19 +1374,7 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
       int ru, rv;
       double cA[4], cB[2];
       block_coefs(w, P, Q, rel == kLocal, cA, cB, ru, rv);
-      // per column direction: the CurlCurl prefactors by row direction (the p
-      // side of the pair is the column's where the source is an ancestor), the
-      // L2Inner prefactor and the library bases
-      double* out = coef + (src_slot(g, n_src) + lane) * kCoef;
-      out[0] = cA[0];
-      out[1] = rel == kAnc ? cA[1] : cA[2];
-      out[4] = rel == kAnc ? cA[2] : cA[1];
-      out[5] = cA[3];
-      const int2 base = make_int2(8 * (ru * w.lib_range_stride), 8 * ((w.lib_nr + rv) * w.lib_range_stride + w.lib_tab));
-      for (int d = 0; d < 2; ++d) {
-        out[4 * d + 2] = cB[d];
-        *reinterpret_cast<int2*>(out + 4 * d + 3) = base;
-      }
+      write_source(w, coef + (src_slot(g, n_src) + lane) * kCoef, cA, cB, ru, rv, rel == kAnc);
       S.src_info[lane] = k | (rel << 1) | (ru << 3) | (rv << 17);
     }
   }
@@ -1387,15 +1385,15 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
   static_assert(kWR == 2 * kWave, "two raw candidates per lane");
   unsigned long long mine[2];
   int rank[2] = {0, 0};
-  for (int h = 0; h < 2; ++h) mine[h] = lane + h * kWave < n_raw ? S.u.sort.key[lane + h * kWave] : ~0ull;
+  for (int h = 0; h < 2; ++h) mine[h] = lane + h * kWave < n_raw ? S.key[lane + h * kWave] : ~0ull;
   for (int k = 0; k < n_raw; ++k) {
-    const unsigned long long kk = S.u.sort.key[k];
+    const unsigned long long kk = S.key[k];
     rank[0] += kk < mine[0] ? 1 : 0;
     rank[1] += kk < mine[1] ? 1 : 0;
   }
   wave_sync();  // every lane has read every key
   for (int h = 0; h < 2; ++h)
-    if (lane + h * kWave < n_raw) S.u.sort.key[rank[h]] = mine[h];
+    if (lane + h * kWave < n_raw) S.key[rank[h]] = mine[h];
   wave_sync();
   // dedupe: first pass writes every new row group, second the second sources
   int running = 0;
@@ -1403,9 +1401,9 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
   for (int base = 0; base < n_raw; base += kWave) {
     const int t = base + lane;
     const bool valid = t < n_raw;
-    const unsigned long long kt = valid ? S.u.sort.key[t] : 0ull;
+    const unsigned long long kt = valid ? S.key[t] : 0ull;
     const int h = valid ? int(kt >> 20) : -1;
-    const int hp = (valid && t > 0) ? int(S.u.sort.key[t - 1] >> 20) : -2;
+    const int hp = (valid && t > 0) ? int(S.key[t - 1] >> 20) : -2;
     const bool is_new = valid && h != hp;
     const unsigned long long mask = __ballot(is_new);
     const unsigned long long upto = lane == kWave - 1 ? ~0ull : ((2ull << lane) - 1ull);
@@ -1415,14 +1413,14 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
       const int gs = w.g_start[h];
       S.dstart[didx] = gs;
       S.cum[didx] = w.g_start[h + 1] - gs;  // size, prefix-summed below
-      S.dmeta0[didx] = S.u.sort.raw_meta[int(kt & 0xFFFFF)];
+      S.dmeta0[didx] = S.raw_meta[int(kt & 0xFFFFF)];
       S.dmeta1[didx] = -1;
     }
     wave_sync();
     if (valid && !is_new && didx < kWD) {
-      const int hpp = t >= 2 ? int(S.u.sort.key[t - 2] >> 20) : -3;
+      const int hpp = t >= 2 ? int(S.key[t - 2] >> 20) : -3;
       if (hpp == h) bad |= 2;  // a third source for one column
-      S.dmeta1[didx] = S.u.sort.raw_meta[int(kt & 0xFFFFF)];
+      S.dmeta1[didx] = S.raw_meta[int(kt & 0xFFFFF)];
     }
     running += __popcll(mask);
     wave_sync();
@@ -1498,66 +1496,349 @@ __device__ __forceinline__ uint2 row_variant(unsigned spec, bool anc, int tab) {
 static_assert(8 * (kMaxOrder * (kMaxOrder + 1) + 2 * (kMaxOrder + 1) * (kMaxOrder + 1)) < (1 << 15) && kWS <= 32,
               "library offsets and sources of the fill's records");
 
-// One wavefront per row group: build the candidate set, then write the row
-// lengths and the group's fixed-stride records for the streaming fill:
-// source prefactors and infos, the packed specs of its rows, and for each
-// candidate column t = 0..T-1 of its first row (candidate index u_self + t)
-// the column and the packed specs of its one or two contributions.
-__global__ void __launch_bounds__(kBlock, kLatencyWavesPerSimd) k_describe_wave(DevView v, Work w) {
-  if (*w.err) return;  // an invalid view was detected: nothing below may trust it
-  __shared__ WaveShared shared[kWavesPerBlock];
-  const int lane = threadIdx.x % kWave;
-  const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
-  WaveShared& S = shared[wid];
-  const int n_groups = n_groups_of(w);
-  // static assignment: a shared work counter would serialise on device-scope
-  // atomics, which span the XCDs' separate L2 caches
-  const int stride = gridDim.x * kWavesPerBlock;
-  for (int g = blockIdx.x * kWavesPerBlock + wid; g < n_groups; g += stride) {
-    if (g >= w.meta_cap) {  // more row groups than the view's DoF signatures give
-      if (lane == 0) set_err(w.err, kErrView);
-      break;
+// One row group by a whole wavefront: its header, source records and, for each
+// candidate column t = 0..T-1 of its first row (candidate index u_self + t), the
+// column record of the streaming fill. A group beyond the wave path's limits is
+// listed for the block path.
+__device__ void describe_group(const DevView& v, const Work& w, int g, WaveShared& S, int lane) {
+  const int st = wave_build(v, w, g, S, lane, w.meta_coef + (long long)g * (kWS * kCoef));
+  const int r0 = ld_const(w.g_start, g), r1 = ld_const(w.g_start, g + 1);
+  const int nrows = r1 - r0;
+  if (st == 1) {
+    if (lane == 0) {
+      w.is_large[g] = 1;
+      w.large_list[atomicAdd(w.n_large, 1)] = g;
+      w.meta_hdr[g] = make_int4(-1, nrows, 0, 0);
     }
-    const long long gs = (long long)g * kWS;
-    const int st = wave_build(v, w, g, S, lane, w.meta_coef + gs * kCoef);
-    const int r0 = ld_const(w.g_start, g), r1 = ld_const(w.g_start, g + 1);
-    const int nrows = r1 - r0;
-    if (st == 1) {
-      if (lane == 0) {
-        w.is_large[g] = 1;
-        w.large_list[atomicAdd(w.n_large, 1)] = g;
-        w.meta_hdr[g] = make_int4(-1, nrows, 0, 0);
+  } else if (st == 0) {
+    const int u_self = S.u_self, n_dist = S.n_dist, n_src = S.n_src;  // set by wave_build
+    const int T = S.total - u_self;
+    if (lane == 0) {
+      w.is_large[g] = 0;
+      w.meta_hdr[g] = make_int4(T, nrows, n_src, r0);
+    }
+    for (int t = lane; t < T; t += kWave) {
+      const int u = u_self + t;
+      int a = 0, b = n_dist;  // cum[a] <= u < cum[b]
+      while (b - a > 1) {
+        const int mid = (a + b) >> 1;
+        if (S.cum[mid] <= u) a = mid; else b = mid;
       }
-    } else if (st == 0) {
-      const int u_self = S.u_self, n_dist = S.n_dist, n_src = S.n_src;  // set by wave_build
-      const int T = S.total - u_self;
-      if (lane == 0) {
-        w.is_large[g] = 0;
-        w.meta_hdr[g] = make_int4(T, nrows, n_src, r0);
+      const int within = u - S.cum[a];
+      const int m0 = S.dmeta0[a], m1 = S.dmeta1[a];
+      uint4 rec;
+      rec.x = unsigned(S.dstart[a] + within);
+      const int s0 = m0 & 0xff, s1 = m1 & 0xff;
+      unsigned y0, y1 = 0u;
+      rec.y = col_contrib(s0, S.src_info[s0], w.bs_pack[S.src_bs[s0] + (m0 >> 8) + within], w.lib_tab, y0);
+      rec.z = ~0u;
+      if (m1 >= 0)
+        rec.z = col_contrib(s1, S.src_info[s1], w.bs_pack[S.src_bs[s1] + (m1 >> 8) + within], w.lib_tab, y1);
+      rec.w = y0 | (y1 << 16);
+      w.meta_col[(long long)g * kWC + col_slot(g, T) + t] = rec;
+    }
+  }
+  wave_sync();
+}
+
+// Row groups by the row: the 16 lanes of a row of the wavefront (the unit of the
+// data-parallel-primitive shifts) describe one group, four groups a wavefront.
+// Most groups are small (hp-irregular: 6 sources, 13 memberships and 33 columns in
+// the mean), so a whole wavefront a group left most lanes idle, and its 433 vector
+// instructions a group bound the kernel (70 % of the issue slots).
+constexpr int kRow = 16;
+constexpr int kRowsPerWave = kWave / kRow;
+constexpr int kRowSrc = kRow;     // sources of a group on this path (one a lane)
+constexpr int kRowRaw = 3 * kRow;  // memberships
+
+struct RowShared {
+  unsigned long long key[kRowRaw];  // row group << 20 | raw index
+  int raw_meta[kRowRaw];            // source | bs offset << 8
+  int4 dist[kRowRaw];  // per candidate group: columns before it, first DoF, source | bs offset << 8 of its
+                       // first and second contribution (-1 if none)
+  int2 src[kRowSrc];   // first basis spec of each source; k | rel << 1
+  uint2 cols[kWC / 32];  // .x: bit p: a candidate group starts at column p + 1 of the row group's columns;
+                         // .y: candidate groups that start in the words before, and the group itself
+  int u_self, self;
+  int cols_at;  // the group's first column record, from its slot's start
+};
+
+union DescribeShared {
+  WaveShared wave;
+  RowShared row[kRowsPerWave];
+};
+
+__device__ __forceinline__ unsigned row_ballot(bool x, int row) {
+  return unsigned(__ballot(x) >> (row * kRow)) & ((1u << kRow) - 1u);
+}
+// inclusive prefix sum over the row
+__device__ __forceinline__ int row_incl_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  return x;
+}
+// the value of the row's last lane
+__device__ __forceinline__ int row_last(int x, int lane) { return __shfl(x, lane | (kRow - 1), kWave); }
+
+// Describes the wavefront's row groups g0.. (one a row; act: the lane's row has
+// one). Returns, per lane, whether the row's group has to be described by a whole
+// wavefront instead.
+__device__ bool describe_rows(const DevView& v, const Work& w, int g0, bool act, RowShared* rows, int lane) {
+  const int sl = lane % kRow, row = lane / kRow;
+  const int g = g0 + row;
+  RowShared& S = rows[row];
+  int e1 = -1, e2 = -1, r0 = 0, nrows = 0;
+  if (act) {
+    e1 = w.g_e1[g];
+    e2 = w.g_e2[g];
+    r0 = w.g_start[g];
+    nrows = w.g_start[g + 1] - r0;
+  }
+  int a1 = 0, n1 = 0, a2 = 0, n2 = 0;  // the nested lists of both Elems
+  if (e1 >= 0) {
+    a1 = w.nested_ptr[e1];
+    n1 = w.nested_ptr[e1 + 1] - a1;
+    if (e2 >= 0) {
+      a2 = w.nested_ptr[e2];
+      n2 = w.nested_ptr[e2 + 1] - a2;
+    }
+  }
+  const int n_src = n1 + n2;
+  bool whole = act && n_src > kRowSrc;
+  act = act && !whole;
+  // one source a lane: its Elem and its memberships
+  const bool is_src = act && sl < n_src;
+  int X = 0, info = 0, m0 = 0, cnt = 0;
+  if (is_src) {
+    const int k = sl < n1 ? 0 : 1;
+    const int x = w.nested[k == 0 ? a1 + sl : a2 + (sl - n1)];
+    X = x >> 2;
+    info = k | ((x & 3) << 1);
+    const long long b0 = v.bs_off[X], b1 = v.bs_off[X + 1];
+    m0 = w.mem_idx[b0];
+    cnt = w.mem_idx[b1] - m0;
+    S.src[sl] = make_int2(int(b0), info);
+  }
+  const int incl = row_incl_scan(cnt);
+  const int n_raw = row_last(incl, lane);
+  if (act && n_raw > kRowRaw) {
+    whole = true;
+    act = false;
+  }
+#pragma unroll
+  for (int h = 0; h < kRowRaw / kRow; ++h) S.key[h * kRow + sl] = ~0ull;
+  if (sl == 0) S.self = -1;
+  if (sl < kWC / 32) S.cols[sl].x = 0u;
+  wave_sync();
+  // raw candidates: each source's memberships, the first four of a lane together
+  const int base = incl - cnt;
+  auto put = [&](int i, int group, int off) {
+    S.key[base + i] = ((unsigned long long)unsigned(group) << 20) | unsigned(base + i);
+    S.raw_meta[base + i] = sl | (off << 8);
+  };
+  if (!act) cnt = 0;
+  {
+    int mg[4], mo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < cnt) {
+        mg[i] = w.mem_group[m0 + i];
+        mo[i] = w.mem_bsoff[m0 + i];
       }
-      for (int t = lane; t < T; t += kWave) {
-        const int u = u_self + t;
-        int a = 0, b = n_dist;  // cum[a] <= u < cum[b]
-        while (b - a > 1) {
-          const int mid = (a + b) >> 1;
-          if (S.cum[mid] <= u) a = mid; else b = mid;
-        }
-        const int within = u - S.cum[a];
-        const int m0 = S.dmeta0[a], m1 = S.dmeta1[a];
-        uint4 rec;
-        rec.x = unsigned(S.dstart[a] + within);
-        const int s0 = m0 & 0xff, s1 = m1 & 0xff;
-        unsigned y0, y1 = 0u;
-        rec.y = col_contrib(s0, S.src_info[s0], w.bs_pack[S.src_bs[s0] + (m0 >> 8) + within], w.lib_tab, y0);
-        rec.z = ~0u;
-        if (m1 >= 0)
-          rec.z = col_contrib(s1, S.src_info[s1], w.bs_pack[S.src_bs[s1] + (m1 >> 8) + within], w.lib_tab, y1);
-        rec.w = y0 | (y1 << 16);
-        w.meta_col[(long long)g * kWC + col_slot(g, T) + t] = rec;
-      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < cnt) put(i, mg[i], mo[i]);
+    for (int i = 4; i < cnt; ++i) put(i, w.mem_group[m0 + i], w.mem_bsoff[m0 + i]);
+  }
+  if (is_src && act) {
+    const int k = info & 1, rel = info >> 1;
+    const int E = k == 0 ? e1 : e2;
+    int ru, rv;
+    double cA[4], cB[2];
+    block_coefs(w, rel == kAnc ? X : E, rel == kAnc ? E : X, rel == kLocal, cA, cB, ru, rv);
+    write_source(w, w.meta_coef + ((long long)g * kWS + src_slot(g, n_src) + sl) * kCoef, cA, cB, ru, rv, rel == kAnc);
+  }
+  wave_sync();  // every raw key is in LDS
+  // rank sort by (row group, gather order), as wave_build's
+  int most = 0;  // raw candidates of the largest of the four
+#pragma unroll
+  for (int i = 0; i < kRowsPerWave; ++i) most = max(most, __builtin_amdgcn_readlane(act ? n_raw : 0, i * kRow));
+  unsigned long long mine[kRowRaw / kRow];
+  int rank[kRowRaw / kRow] = {};
+#pragma unroll
+  for (int h = 0; h < kRowRaw / kRow; ++h) mine[h] = S.key[h * kRow + sl];
+  for (int k = 0; k < most; ++k) {
+    const unsigned long long kk = S.key[k];
+    rank[0] += kk < mine[0] ? 1 : 0;
+    if (most > kRow) {
+      rank[1] += kk < mine[1] ? 1 : 0;
+      rank[2] += kk < mine[2] ? 1 : 0;
+    }
+  }
+  wave_sync();  // every lane has read every key
+#pragma unroll
+  for (int h = 0; h < kRowRaw / kRow; ++h)
+    if (act && h * kRow + sl < n_raw) S.key[rank[h]] = mine[h];
+  wave_sync();
+  // dedupe: the distinct row groups with their first and second contributions
+  int n_dist = 0;
+  bool bad = false;
+  for (int h = 0; h * kRow < most; ++h) {
+    const int t = h * kRow + sl;
+    const bool in = act && t < n_raw;
+    const unsigned long long kt = in ? S.key[t] : 0ull;
+    const int c = in ? int(kt >> 20) : -1;
+    const int cp = in && t > 0 ? int(S.key[t - 1] >> 20) : -2;
+    const bool is_new = in && c != cp;
+    const unsigned news = row_ballot(is_new, row);
+    const int d = n_dist + __popc(news & ((2u << sl) - 1u)) - 1;
+    if (is_new) {
+      const int gs = w.g_start[c];
+      S.dist[d] = make_int4(w.g_start[c + 1] - gs, gs, S.raw_meta[int(kt & 0xFFFFF)], -1);
     }
     wave_sync();
+    if (in && !is_new) {
+      if (t >= 2 && int(S.key[t - 2] >> 20) == c) bad = true;  // a third source for one column
+      S.dist[d].w = S.raw_meta[int(kt & 0xFFFFF)];
+    }
+    n_dist += __popc(news);
+    wave_sync();
   }
+  if (row_ballot(bad, row)) {
+    if (bad) set_err(w.err, kErrContrib);
+    act = false;
+  }
+  // columns before each distinct group; the group itself among them
+  int total = 0;
+  for (int h = 0; h * kRow < most; ++h) {
+    const int t = h * kRow + sl;
+    const bool in = act && t < n_dist;
+    const int sz = in ? S.dist[t].x : 0;
+    const int inc = row_incl_scan(sz);
+    if (in) {
+      S.dist[t].x = total + inc - sz;
+      if (S.dist[t].y == r0) {
+        S.u_self = total + inc - sz;
+        S.self = t;
+      }
+    }
+    total += row_last(inc, lane);
+  }
+  wave_sync();
+  const int self = S.self;
+  if (act && self < 0) {  // the group is not among its own candidates
+    if (sl == 0) set_err(w.err, kErrView);
+    act = false;
+  }
+  const int u_self = act ? S.u_self : 0;
+  const int T = act ? total - u_self : 0;
+  if (act && (T > kWC || nrows > kWRows)) {  // the whole wavefront's path lists it for the block path
+    whole = true;
+    act = false;
+  }
+  if (act && sl == 0) {
+    w.is_large[g] = 0;
+    w.meta_hdr[g] = make_int4(T, nrows, n_src, r0);
+  }
+  // the groups' first columns as a bitmap, so that a column finds its group by counting
+  if (act)
+    for (int t = self + 1 + sl; t < n_dist; t += kRow) {
+      const int p = S.dist[t].x - u_self - 1;
+      atomicOr(&S.cols[p >> 5].x, 1u << (p & 31));
+    }
+  wave_sync();
+  {
+    const int c = sl < kWC / 32 ? __popc(S.cols[sl].x) : 0;
+    const int inc = row_incl_scan(c);
+    if (sl < kWC / 32) S.cols[sl].y = unsigned(self + inc - c);
+  }
+  if (sl == 0) S.cols_at = col_slot(g, T);
+  wave_sync();
+  // the columns of the four groups one after another over all lanes, two a lane at
+  // a time so that their loads are in flight together
+  int first[kRowsPerWave + 1] = {0};
+#pragma unroll
+  for (int i = 0; i < kRowsPerWave; ++i) first[i + 1] = first[i] + __builtin_amdgcn_readlane(T, i * kRow);
+  const int n = first[kRowsPerWave];
+  struct Column {
+    const RowShared* S;
+    int row, t, within;
+    int4 c;
+  };
+  auto find = [&](int f) {
+    Column x;
+    x.row = (f >= first[1] ? 1 : 0) + (f >= first[2] ? 1 : 0) + (f >= first[3] ? 1 : 0);
+    x.t = f - (x.row == 0 ? 0 : x.row == 1 ? first[1] : x.row == 2 ? first[2] : first[3]);
+    x.S = rows + x.row;
+    const uint2 word = x.S->cols[x.t >> 5];
+    x.c = x.S->dist[word.y + __popc(word.x & ((1u << (x.t & 31)) - 1u))];
+    x.within = x.S->u_self + x.t - x.c.x;
+    return x;
+  };
+  auto spec = [&](const Column& x, int meta) { return w.bs_pack[x.S->src[meta & 0xff].x + (meta >> 8) + x.within]; };
+  auto put_column = [&](const Column& x, unsigned p0, unsigned p1) {
+    uint4 rec;
+    rec.x = unsigned(x.c.y + x.within);
+    unsigned y0, y1 = 0u;
+    const int s0 = x.c.z & 0xff, s1 = x.c.w & 0xff;
+    rec.y = col_contrib(s0, x.S->src[s0].y, p0, w.lib_tab, y0);
+    rec.z = ~0u;
+    if (x.c.w >= 0) rec.z = col_contrib(s1, x.S->src[s1].y, p1, w.lib_tab, y1);
+    rec.w = y0 | (y1 << 16);
+    w.meta_col[(long long)(g0 + x.row) * kWC + x.S->cols_at + x.t] = rec;
+  };
+  for (int f = lane; f < n; f += 2 * kWave) {
+    const bool two = f + kWave < n;
+    const Column a = find(f), b = find(two ? f + kWave : f);
+    const unsigned a0 = spec(a, a.c.z), b0 = spec(b, b.c.z);
+    const unsigned a1 = a.c.w >= 0 ? spec(a, a.c.w) : 0u, b1 = b.c.w >= 0 ? spec(b, b.c.w) : 0u;
+    put_column(a, a0, a1);
+    if (two) put_column(b, b0, b1);
+  }
+  wave_sync();  // every lane is done with the rows' LDS
+  return whole;
+}
+
+// The row groups' records for the streaming fill: headers, source records and
+// column records (the rows' packed specs are written by the DoF-group scan).
+__global__ void __launch_bounds__(kBlock, kDescribeWavesPerSimd) k_describe(DevView v, Work w) {
+  if (*w.err) return;  // an invalid view was detected: nothing below may trust it
+  __shared__ DescribeShared shared[kWavesPerBlock];
+  const int lane = threadIdx.x % kWave;
+  const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
+  DescribeShared& S = shared[wid];
+  const int n_groups = n_groups_of(w);
+  // more row groups than the view's DoF signatures give have no room for records
+  if (n_groups > w.meta_cap && blockIdx.x == 0 && threadIdx.x == 0) set_err(w.err, kErrView);
+  const int n = min(n_groups, w.meta_cap);
+  // groups that need a whole wavefront are shared out over the block's wavefronts at
+  // the end: they come in clusters (the edges of one much refined Elem), and four
+  // of them one after another on the wavefront that met them ended the kernel 10 us late
+  constexpr int kList = 128;
+  __shared__ int list[kList], n_list;
+  if (threadIdx.x == 0) n_list = 0;
+  __syncthreads();
+  // static assignment: a shared work counter would serialise on device-scope
+  // atomics, which span the XCDs' separate L2 caches
+  const int stride = gridDim.x * kWavesPerBlock * kRowsPerWave;
+  for (int g0 = (blockIdx.x * kWavesPerBlock + wid) * kRowsPerWave; g0 < n; g0 += stride) {
+    bool whole = describe_rows(v, w, g0, g0 + lane / kRow < n, S.row, lane) && lane % kRow == 0;
+    if (whole) {
+      const int i = atomicAdd(&n_list, 1);
+      if (i < kList) {
+        list[i] = g0 + lane / kRow;
+        whole = false;
+      }
+    }
+    for (unsigned long long left = __ballot(whole); left; left &= left - 1)  // the list is full
+      describe_group(v, w, g0 + __builtin_ctzll(left) / kRow, S.wave, lane);
+  }
+  __syncthreads();
+  const int n_whole = min(n_list, kList);
+  for (int i = wid; i < n_whole; i += kWavesPerBlock)
+    describe_group(v, w, __builtin_amdgcn_readfirstlane(list[i]), S.wave, lane);
 }
 
 __device__ __forceinline__ void write_entry(const FillOut& o, long long pos, int c, double cc, double l2) {
@@ -2953,7 +3234,7 @@ int launch_prep(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, long long* st
   if (fine_events) HIP_TRY(hipEventRecord(ctx->ev[1], st));
   // symbolic: per-group candidate sets, row lengths and records, then row_ptr
   if (fine_events) HIP_TRY(hipEventRecord(ctx->ev[4], st));
-  k_describe_wave<<<unsigned(ctx->count_grid), kBlock, 0, st>>>(v, w);
+  k_describe<<<unsigned(ctx->count_grid), kBlock, 0, st>>>(v, w);
   if (fine_events) HIP_TRY(hipEventRecord(ctx->ev[5], st));
   const unsigned large_grid = unsigned(std::max(1, ctx->n_cu * 2));
   if (a.run_large) k_count_large<<<large_grid, kBlock, sizeof(GroupShared), st>>>(v, w);
@@ -3151,7 +3432,7 @@ int fem2d_ctx_create(int device, fem2d_ctx** out) {
   // the wave kernels assign row groups statically: launch exactly the blocks
   // that are resident at once
   int per_cu = 0;
-  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_describe_wave, kBlock, 0));
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_describe, kBlock, 0));
   ctx->count_grid = std::max(1, per_cu) * ctx->n_cu;
   if (int rc = fill_grids<FEM2D_PRECISION_FP64>(ctx)) return rc;
   if (int rc = fill_grids<FEM2D_PRECISION_FP32>(ctx)) return rc;
