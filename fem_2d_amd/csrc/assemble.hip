@@ -2828,6 +2828,7 @@ struct fem2d_ctx {
   int fill_chunk = 0;  // fill chunk size forced for every assembly (0: fill_chunk_of's)
   hipGraphExec_t graph_exec[1] = {nullptr};  // the last recorded assembly
   GraphKey graph_key;
+  GraphKey last_key;  // of the latest assembly: only the second in a row of a key is recorded
   void* solver = nullptr;  // eigensolver handle, made by the first solve
   // generation of the latest assembly whose outputs the buffers hold (0: none)
   unsigned long long out_generation = 0;
@@ -3705,8 +3706,8 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
   // The assembly in three parts: (a) preparation and symbolic phase, ending
   // with the CSR layout and the status block, (b) the streaming fill, (c) the
   // block-path fill (only for Domains with large row groups). With graphs the
-  // three are recorded as one graph, replayed while the Domain, the options
-  // and the buffers stay the same, and timed end to end; kernel by kernel,
+  // three are recorded as one graph the second time in a row that they come with the same
+  // Domain, options and buffers, replayed while these stay, and timed end to end; kernel by kernel,
   // events between the stages also time the stages and the describe and fill
   // kernels on their own.
   // record the work of parts() into ctx->graph_exec[i]
@@ -3748,30 +3749,40 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
     if (ctx->use_graphs) {
       const GraphKey key{dd->serial, basis,     ai,       bi, nu, nv, o.capacity, g_alloc_generation.load(),
                          run_large,  precision, w.chunk};
-      if (!ctx->graph_exec[0] || !(key == ctx->graph_key)) {
+      auto whole = [&]() -> int {
+        int prc = launch_prep(ctx, st, a, ctx->d_status, false);
+        if (prc != FEM2D_OK) return prc;
+        // the block-path fill writes segments of its own, from row pointers the
+        // layout scan wrote: a branch beside the streaming fill (a branch
+        // costs the graph ~20 us, so only this one)
+        if (tail) {
+          HIP_TRY(hipEventRecord(ctx->fork_ev, st));
+          HIP_TRY(hipStreamWaitEvent(ctx->side_stream, ctx->fork_ev, 0));
+          if ((prc = launch_large_fill(ctx, ctx->side_stream, a, o))) return prc;
+          HIP_TRY(hipEventRecord(ctx->join_ev, ctx->side_stream));
+        }
+        if (fill && (prc = launch_stream_fill(ctx, st, a, o))) return prc;
+        if (tail) HIP_TRY(hipStreamWaitEvent(st, ctx->join_ev, 0));
+        return prc;
+      };
+      const bool recorded = ctx->graph_exec[0] && key == ctx->graph_key;
+      if (!recorded && key == ctx->last_key) {
         ctx->graph_key = GraphKey{};
-        if ((rc = record(0, [&] {
-               int prc = launch_prep(ctx, st, a, ctx->d_status, false);
-               if (prc != FEM2D_OK) return prc;
-               // the block-path fill writes segments of its own, from row
-               // pointers the layout scan wrote: a branch beside the streaming
-               // fill (a branch costs the graph ~20 us, so only this one)
-               if (tail) {
-                 HIP_TRY(hipEventRecord(ctx->fork_ev, st));
-                 HIP_TRY(hipStreamWaitEvent(ctx->side_stream, ctx->fork_ev, 0));
-                 if ((prc = launch_large_fill(ctx, ctx->side_stream, a, o))) return prc;
-                 HIP_TRY(hipEventRecord(ctx->join_ev, ctx->side_stream));
-               }
-               if (fill && (prc = launch_stream_fill(ctx, st, a, o))) return prc;
-               if (tail) HIP_TRY(hipStreamWaitEvent(st, ctx->join_ev, 0));
-               return prc;
-             })))
-          return rc;
+        if ((rc = record(0, whole))) return rc;
         ctx->graph_key = key;
       }
-      // one graph for the whole assembly; only its end points are timed
+      // only the end points of the whole assembly are timed
       HIP_TRY(hipEventRecord(ctx->ev[0], st));
-      HIP_TRY(hipGraphLaunch(ctx->graph_exec[0], st));
+      if (key == ctx->graph_key) {
+        HIP_TRY(hipGraphLaunch(ctx->graph_exec[0], st));
+      } else {
+        // not the same Domain, options and buffers as the assembly before: a Domain of
+        // an adaptive loop or of a drop-in call is assembled only once, and a
+        // recording costs more than the launches it saves (the assembly of a new
+        // hp-irregular 32 x 16 Domain 310 us recorded and replayed, 177 launched)
+        if ((rc = whole())) return rc;
+      }
+      ctx->last_key = key;
       HIP_TRY(hipEventRecord(ctx->ev[3], st));
       fine_timing = false;
     } else {

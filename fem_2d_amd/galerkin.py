@@ -90,7 +90,8 @@ class Context:
             pass
 
     def set_graphs(self, enable: bool) -> None:
-        """Record each assembly once as a HIP graph and replay it (default), or launch kernel by kernel."""
+        """Record an assembly that is repeated as a HIP graph and replay it (default), or launch kernel
+        by kernel."""
         check(self._lib.fem2d_ctx_set_graphs(self._h, 1 if enable else 0))
 
     def set_autotune(self, enable: bool) -> None:

@@ -149,8 +149,9 @@ void fem2d_ctx_destroy(fem2d_ctx* ctx);
 void* fem2d_ctx_stream(fem2d_ctx* ctx);
 /* device-wide synchronisation of the context's device */
 int fem2d_ctx_synchronize(fem2d_ctx* ctx);
-/* Whether assemblies on this context are recorded once as a HIP graph and
- * replayed (default 1) or launched kernel by kernel (0). Results are the same;
+/* Whether assemblies on this context are recorded as a HIP graph, the second time
+ * in a row that one Domain comes with the same options and buffers, and replayed
+ * (default 1) or launched kernel by kernel (0). Results are the same;
  * graphs remove the per-kernel launch gaps of the ~20-kernel pipeline. */
 int fem2d_ctx_set_graphs(fem2d_ctx* ctx, int enable);
 /* Accepted for callers of earlier versions, which timed the entry fill's shapes on a

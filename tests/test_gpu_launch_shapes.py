@@ -1,0 +1,88 @@
+"""Sizes at which the assembly and field kernels change their split of the work: the describe
+kernel's two ways to share out row groups (a wavefront or sixteen lanes each, with the groups of many
+sources shared by a block), the one- and two-pass CSR layout, the fill's chunks, the field grid's
+tiles of 16 points, and an assembly's recording as a graph on its second call in a row. GEPs within
+_compare.RTOL of the oracle, fields within 1e-13 of the largest (as in the fields' other tests);
+forced chunks and graph replays give the same bits."""
+
+import numpy as np
+import pytest
+
+import cases
+import fem_2d_amd as F
+import oracle
+from _compare import assert_gep_matches
+from fem_2d_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+FIELD_TOL = 1e-13
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return F.Context(0)
+
+
+def _same_bits(g, ref):
+    np.testing.assert_array_equal(g.row_ptr, ref.row_ptr)
+    np.testing.assert_array_equal(g.col, ref.col)
+    np.testing.assert_array_equal(g.a_val.view(np.uint8), ref.a_val.view(np.uint8))
+    np.testing.assert_array_equal(g.b_val.view(np.uint8), ref.b_val.view(np.uint8))
+
+
+# 1, 2 190 (past the 2 048 where the layout takes its second pass), 4 163, 17 080 and 29 527 groups (the
+# last two past two groups a wavefront); 16, 14, 49 and 513 of them have more than 16 sources
+@pytest.mark.parametrize("nx,ny,levels", [(1, 1, 0), (22, 12, 2), (32, 16, 2), (64, 32, 2), (64, 32, 3)])
+def test_row_groups(ctx, nx, ny, levels):
+    print(f"[shapes] waveguide {nx}x{ny} levels={levels}", flush=True)
+    dom = F.Domain.from_mesh(W.waveguide_64x32_mesh(nx, ny, order=2, levels=levels))
+    gep = F.galerkin_sample_gep_hcurl(dom, (8, 8), F.HierPoly, ctx=ctx)
+    rc, ref = oracle.assemble(dom.view(), basis=F.HierPoly.code, glq=(8, 8), n_threads=8)
+    assert rc == 0
+    assert_gep_matches(gep, ref)
+
+
+@pytest.mark.parametrize("name", ["waveguide_small", "small_hp_irregular", "deep_corner"])
+def test_forced_chunks(ctx, name):
+    dom, glq = cases.ALL[name]()
+    ref = F.galerkin_sample_gep_hcurl(dom, glq, F.KOLShapeFn, ctx=ctx)
+    c = F.Context(0)
+    for chunk in (64, 128, 1024, 4096):
+        print(f"[shapes] {name} chunk={chunk}", flush=True)
+        c.set_fill_chunk(chunk)
+        _same_bits(F.galerkin_sample_gep_hcurl(dom, glq, F.KOLShapeFn, ctx=c), ref)
+    c.close()
+
+
+@pytest.mark.parametrize("basis", [0, 1])
+@pytest.mark.parametrize("d", [2, 15, 16, 17, 33])
+def test_field_tiles(ctx, basis, d):
+    """A NaN DoF value reaches the points that it reaches in the oracle's sums."""
+    print(f"[shapes] fields basis={basis} d={d}", flush=True)
+    dom, _ = cases.small_hp_irregular()
+    B = F.KOLShapeFn if basis else F.HierPoly
+    sol = np.random.default_rng(d).standard_normal(dom.num_dofs)
+    for poison in (False, True):
+        if poison:
+            sol[dom.num_dofs // 2] = np.nan
+        rc, ex, ey = oracle.xy_fields(dom.view(), basis, (d, d), sol)
+        assert rc == 0
+        for got, exp in zip(F.xy_fields_array(dom, sol, (d, d), B, ctx=ctx), (ex, ey)):
+            np.testing.assert_array_equal(np.isnan(got), np.isnan(exp))
+            assert np.nanmax(np.abs(got - exp)) <= FIELD_TOL * np.nanmax(np.abs(exp))
+
+
+def test_recording_order():
+    """Launched, recorded and replayed assemblies of two Domains of one context in every order of
+    succession, the second one's larger buffers allocated after the first one's recording."""
+    print("[shapes] recording order", flush=True)
+    c, eager = F.Context(0), F.Context(0)
+    eager.set_graphs(False)
+    made = [cases.waveguide_small(), cases.small_hp_irregular()]
+    refs = [F.galerkin_sample_gep_hcurl(d, q, F.HierPoly, ctx=eager) for d, q in made]
+    doms = [F.DeviceDomain(d, c) for d, _ in made]
+    for i in (0, 0, 0, 1, 0, 1, 1, 1, 0, 1, 0, 0, 0, 1):
+        _same_bits(doms[i].download(doms[i].assemble(made[i][1], F.HierPoly)), refs[i])
+    c.close()
+    eager.close()
