@@ -275,7 +275,7 @@ __global__ void k_lu_apply(long long n, const double* __restrict__ X, const int*
 // filled alike: the column dots, one wavefront a column, contiguous and with four
 // loads in flight a lane. A solve of 1 096 DoFs has 81 of these products, 47 us each as a
 // library matrix-vector product; the whole solve 20.2 -> 14.8 ms, 606 DoFs 10.9 -> 8.9,
-// 4 496 DoFs 107.9 -> 103.6.
+// 4 496 DoFs (mean of 12 targets) 133 -> 127.
 __global__ void k_sym_mv(long long n, const double* __restrict__ M, const double* __restrict__ x,
                          const double* __restrict__ b, double* __restrict__ y) {
   const int lane = threadIdx.x % kWave;
@@ -294,6 +294,79 @@ __global__ void k_sym_mv(long long n, const double* __restrict__ M, const double
     for (; r < n; r += kWave) s0 += col[r] * x[r];
     const double s = wave_sum((s0 + s1) + (s2 + s3));
     if (lane == 0) y[c] = b ? b[c] - s : s;
+  }
+}
+
+// The iteration's reductions, by one block: the vectors are at most 32 768 long and a
+// solve of 1 096 DoFs has a hundred of them, each a library call of two kernels, a
+// copy and a host wait before. Scalars that are needed together are read together.
+// 1 096 DoFs 14.8 -> 12.8 ms, 606 DoFs 8.9 -> 7.1; from 3 430 on within 1 %.
+constexpr int kSolo = 1024;
+
+// sum over the block of kSolo threads (every thread receives it)
+__device__ __forceinline__ double solo_sum(double x, double* sums) {
+  x = wave_sum(x);
+  __syncthreads();  // the readers of an earlier sum are done
+  if (threadIdx.x % kWave == 0) sums[threadIdx.x / kWave] = x;
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < kSolo / kWave; ++k) s += sums[k];
+  return s;
+}
+
+// out[0] = |r|, out[1] = |b|
+__global__ void __launch_bounds__(kSolo) k_two_norms(int n, const double* __restrict__ r, const double* __restrict__ b,
+                                                     double* __restrict__ out) {
+  __shared__ double sums[kSolo / kWave];
+  double sr = 0.0, sb = 0.0;
+  for (int i = threadIdx.x; i < n; i += kSolo) {
+    sr += r[i] * r[i];
+    sb += b[i] * b[i];
+  }
+  sr = solo_sum(sr, sums);
+  sb = solo_sum(sb, sums);
+  if (threadIdx.x == 0) {
+    out[0] = sqrt(sr);
+    out[1] = sqrt(sb);
+  }
+}
+
+// out[0] = s = y . by; x = y / sqrt(s), bx = by / sqrt(s) (by and bx may be the same)
+__global__ void __launch_bounds__(kSolo) k_normalise(int n, const double* __restrict__ y, const double* by, double* x,
+                                                     double* bx, double* __restrict__ out) {
+  __shared__ double sums[kSolo / kWave];
+  double s = 0.0;
+  for (int i = threadIdx.x; i < n; i += kSolo) s += y[i] * by[i];
+  s = solo_sum(s, sums);
+  if (threadIdx.x == 0) out[0] = s;
+  const double inv = 1.0 / sqrt(s);
+  for (int i = threadIdx.x; i < n; i += kSolo) {
+    x[i] = y[i] * inv;
+    bx[i] = by[i] * inv;
+  }
+}
+
+// out[1] = lambda = x . ax, out[2] = |ax|, out[3] = |ax - lambda bx|
+__global__ void __launch_bounds__(kSolo) k_rayleigh(int n, const double* __restrict__ x, const double* __restrict__ ax,
+                                                    const double* __restrict__ bx, double* __restrict__ out) {
+  __shared__ double sums[kSolo / kWave];
+  double l = 0.0, a = 0.0, e = 0.0;
+  for (int i = threadIdx.x; i < n; i += kSolo) {
+    l += x[i] * ax[i];
+    a += ax[i] * ax[i];
+  }
+  l = solo_sum(l, sums);
+  a = solo_sum(a, sums);
+  for (int i = threadIdx.x; i < n; i += kSolo) {
+    const double v = ax[i] - l * bx[i];
+    e += v * v;
+  }
+  e = solo_sum(e, sums);
+  if (threadIdx.x == 0) {
+    out[1] = l;
+    out[2] = sqrt(a);
+    out[3] = sqrt(e);
   }
 }
 
@@ -435,6 +508,14 @@ int inverse_iteration(rocblas_handle h, hipStream_t st, long long n, const doubl
     EIG_HIP(hipGetLastError());
     return FEM2D_OK;
   };
+  double* scalars;  // the iterate's s, lambda, |A x|, |A x - lambda B x|; or two norms
+  EIG_HIP(m.alloc(&scalars, 4));
+  auto read_scalars = [&](int count, double* out) -> int {
+    EIG_HIP(hipGetLastError());
+    EIG_HIP(hipMemcpyAsync(out, scalars, size_t(count) * sizeof(double), hipMemcpyDeviceToHost, st));
+    EIG_HIP(hipStreamSynchronize(st));
+    return FEM2D_OK;
+  };
   if (int rc = product(B, x, nullptr, bx)) return rc;
   // converged: a relative residual |A x - lambda B x| / |A x| of kTol, or of
   // kTolStall once the Rayleigh quotient no longer moves (the residual's
@@ -449,7 +530,6 @@ int inverse_iteration(rocblas_handle h, hipStream_t st, long long n, const doubl
     // conditioning. A solve the refinement leaves inaccurate (the first
     // iteration shows it) switches every later solve to getrs.
     double nb = 0.0;
-    if (!exact) EIG_BLAS(rocblas_dnrm2(h, ni, bx, 1, &nb));
     for (int attempt = 0; attempt < 2; ++attempt) {
       if (int rc = lu_solve(bx, y)) return rc;
       double nres = HUGE_VAL, nr_prev = HUGE_VAL;
@@ -459,7 +539,11 @@ int inverse_iteration(rocblas_handle h, hipStream_t st, long long n, const doubl
         if (exact && k == steps) break;
         if (int rc = product(K0, y, bx, r)) return rc;  // B x - K y
         if (!exact) {
-          EIG_BLAS(rocblas_dnrm2(h, ni, r, 1, &nres));
+          double norms[2];
+          k_two_norms<<<1, kSolo, 0, st>>>(int(n), r, bx, scalars);
+          if (int rc = read_scalars(2, norms)) return rc;
+          nres = norms[0];
+          nb = norms[1];
           if (k == steps || !(nres > 1e-15 * nb) || !(nres < 0.5 * nr_prev)) break;
           nr_prev = nres;
         }
@@ -473,21 +557,14 @@ int inverse_iteration(rocblas_handle h, hipStream_t st, long long n, const doubl
       exact = true;
     }
     if (int rc = product(B, y, nullptr, bx)) return rc;
-    double s = 0.0;
-    EIG_BLAS(rocblas_ddot(h, ni, y, 1, bx, 1, &s));
-    if (!(s > 0.0) || !std::isfinite(s)) return 1;
-    const double inv = 1.0 / std::sqrt(s);
-    EIG_BLAS(rocblas_dcopy(h, ni, y, 1, x, 1));
-    EIG_BLAS(rocblas_dscal(h, ni, &inv, x, 1));   // x^T B x = 1
-    EIG_BLAS(rocblas_dscal(h, ni, &inv, bx, 1));  // B x
+    k_normalise<<<1, kSolo, 0, st>>>(int(n), y, bx, x, bx, scalars);  // x^T B x = 1
+    EIG_HIP(hipGetLastError());
     if (int rc = product(A, x, nullptr, ax)) return rc;
-    double lam = 0.0, na = 0.0, nr = 0.0;
-    EIG_BLAS(rocblas_ddot(h, ni, x, 1, ax, 1, &lam));
-    EIG_BLAS(rocblas_dnrm2(h, ni, ax, 1, &na));
-    const double neg = -lam;
-    EIG_BLAS(rocblas_dcopy(h, ni, ax, 1, y, 1));
-    EIG_BLAS(rocblas_daxpy(h, ni, &neg, bx, 1, y, 1));  // A x - lambda B x
-    EIG_BLAS(rocblas_dnrm2(h, ni, y, 1, &nr));
+    k_rayleigh<<<1, kSolo, 0, st>>>(int(n), x, ax, bx, scalars);
+    double got[4];
+    if (int rc = read_scalars(4, got)) return rc;
+    const double s = got[0], lam = got[1], na = got[2], nr = got[3];
+    if (!(s > 0.0) || !std::isfinite(s)) return 1;
     if (!std::isfinite(lam) || !std::isfinite(nr)) return 1;
     const bool stalled = std::fabs(lam - lam_prev) <= 1e-14 * std::fabs(lam);
     lam_prev = lam;
