@@ -27,11 +27,11 @@
 //    most two nested pairs, so an entry has one or two contributions; they are
 //    summed in a fixed order and written once. Kernels check this bound and
 //    report a violation instead of writing wrong values.
-//  * One wavefront owns one row group: it builds the candidate set in its own
-//    slice of LDS with wave-level scans, a bitonic sort and ballots (no block
-//    barriers), then streams the group's rows with consecutive lanes on
-//    consecutive CSR slots. Row groups whose candidate set exceeds the wave
-//    slice go to a block-per-group path with a larger LDS budget.
+//  * Sixteen lanes or a whole wavefront describe a row group: its candidate set, by
+//    scans, a sort and ballots in LDS, and the records its entries are made of. The
+//    fill streams the CSR in chunks, consecutive lanes on consecutive slots
+//    whatever the groups. Row groups whose candidate set exceeds the wave's slice
+//    go to a block-per-group path with a larger LDS budget.
 //  * Pattern (count pass + scan) and values (fill pass) are computed on the
 //    device in the same call. The only host synchronisation is at the end (or
 //    when the output buffers must grow).
