@@ -2727,6 +2727,57 @@ __global__ void __launch_bounds__(kWave, kFieldWavesPerSimd) k_xy_fields(DevView
   }
 }
 
+// The same sums for a Domain with orders above kMaxOrder (a Mesh has none; a view
+// filled by hand may), which packed specs cannot hold: one thread a point, the
+// specs one by one from the unpacked arrays, each product formed in the
+// reference's order: (jac_inv row * shape) * shape, then * DoF value.
+template <int kBasis>
+__global__ void __launch_bounds__(kBlock) k_xy_fields_any(DevView v, const ElemGeo* __restrict__ geo,
+                                                          const int4* __restrict__ dyad,
+                                                          const int* __restrict__ leaves, long long n_leaves, int d,
+                                                          double step, const double* __restrict__ sol,
+                                                          double* __restrict__ fx, double* __restrict__ fy) {
+  const long long per_leaf = (long long)d * d;
+  const long long total = n_leaves * per_leaf;
+  for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
+       idx += (long long)gridDim.x * blockDim.x) {
+    const int leaf = leaves[idx / per_leaf];
+    const int4 at = dyad[leaf];
+    const double px = double(int((idx / d) % d)) * step + -1.0, py = double(int(idx % d)) * step + -1.0;
+    double sx = 0.0, sy = 0.0;
+    for (int A = leaf; A >= 0; A = v.parent[A]) {
+      const int4 up = dyad[A];
+      const ElemGeo g = geo[A];
+      const double jz = -0.0;
+      double x = px, y = py;
+      if (A != leaf) {  // the leaf takes the points as given
+        double s, c;
+        range_of(range_key(at.x - up.x, at.y - (up.y << (at.x - up.x))), s, c);
+        x = x * s + c;
+        range_of(range_key(at.z - up.z, at.w - (up.w << (at.z - up.z))), s, c);
+        y = y * s + c;
+      }
+      for (long long t = v.bs_off[A]; t < v.bs_off[A + 1]; ++t) {
+        const double value = sol[v.bs_dof[t]];
+        double Nu, Ndu, Tu, Tdu, Nv, Ndv, Tv, Tdv;
+        if (kBasis == FEM2D_BASIS_KOL) {
+          kol(v.bs_i[t], x, Nu, Ndu, Tu, Tdu);
+          kol(v.bs_j[t], y, Nv, Ndv, Tv, Tdv);
+        } else {
+          hier_poly(v.bs_i[t], x, Nu, Ndu, Tu, Tdu);
+          hier_poly(v.bs_j[t], y, Nv, Ndv, Tv, Tdv);
+        }
+        const bool u = v.bs_dir[t] == FEM2D_DIR_U;
+        const double a = u ? Nu : Tu, b = u ? Tv : Nv;
+        sx += (((u ? g.ju0 : jz) * a) * b) * value;
+        sy += (((u ? jz : g.jv1) * a) * b) * value;
+      }
+    }
+    fx[idx] = sx;
+    fy[idx] = sy;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
@@ -4018,15 +4069,20 @@ int fem2d_device_xy_fields(fem2d_ctx* ctx, const fem2d_device_domain* dd, int ba
   // uniform_range(-1.0, 1.0, d) (fields.rs:402-405): point i is i step - 1
   const double step = (1.0 - -1.0) / double(d - 1);
   const DevView v = dev_view(dd);
-  const long long tiles = (d + kFieldTile - 1) / kFieldTile;
-  const unsigned grid = unsigned(std::min<long long>(dd->n_leaves * tiles * tiles, std::max(1, ctx->n_cu) * 128LL));
-  const size_t lds = field_lds_bytes(v.p1);
-  if (basis == FEM2D_BASIS_KOL)
-    k_xy_fields<FEM2D_BASIS_KOL><<<grid, kWave, lds, ctx->stream>>>(v, dd->geo, dd->dyad, dd->bs_pack, dd->leaves,
-                                                                   dd->n_leaves, d, step, solution, out_x, out_y);
-  else
-    k_xy_fields<FEM2D_BASIS_HIERPOLY><<<grid, kWave, lds, ctx->stream>>>(
-        v, dd->geo, dd->dyad, dd->bs_pack, dd->leaves, dd->n_leaves, d, step, solution, out_x, out_y);
+  const bool kol = basis == FEM2D_BASIS_KOL;
+  const int cus = std::max(1, ctx->n_cu);
+  if (v.p1 > kMaxOrder + 1) {
+    const unsigned grid = unsigned(std::min<long long>((total + kBlock - 1) / kBlock, cus * 16LL));
+    auto* kernel = kol ? k_xy_fields_any<FEM2D_BASIS_KOL> : k_xy_fields_any<FEM2D_BASIS_HIERPOLY>;
+    kernel<<<grid, kBlock, 0, ctx->stream>>>(v, dd->geo, dd->dyad, dd->leaves, dd->n_leaves, d, step, solution, out_x,
+                                             out_y);
+  } else {
+    const long long tiles = (d + kFieldTile - 1) / kFieldTile;
+    const unsigned grid = unsigned(std::min<long long>(dd->n_leaves * tiles * tiles, cus * 128LL));
+    auto* kernel = kol ? k_xy_fields<FEM2D_BASIS_KOL> : k_xy_fields<FEM2D_BASIS_HIERPOLY>;
+    kernel<<<grid, kWave, field_lds_bytes(v.p1), ctx->stream>>>(v, dd->geo, dd->dyad, dd->bs_pack, dd->leaves,
+                                                                dd->n_leaves, d, step, solution, out_x, out_y);
+  }
   HIP_TRY_AT(hipGetLastError(), "after the field kernel");
   HIP_TRY_AT(hipStreamSynchronize(ctx->stream), "after the field kernel");
   return FEM2D_OK;

@@ -5,6 +5,8 @@ tiles of 16 points, and an assembly's recording as a graph on its second call in
 _compare.RTOL of the oracle, fields within 1e-13 of the largest (as in the fields' other tests);
 forced chunks and graph replays give the same bits."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 import scipy.linalg
@@ -13,7 +15,9 @@ import cases
 import fem_2d_amd as F
 import oracle
 from _compare import assert_gep_matches
+from fem_2d_amd import _native as N
 from fem_2d_amd import workloads as W
+from test_gpu_parity import _view_from_arrays
 
 pytestmark = pytest.mark.gpu
 
@@ -105,3 +109,27 @@ def test_solve_of_few_dofs(ctx, nx, ny, order, solve):
     x = pair.vector
     assert abs(pair.value - lam) <= 1e-10 * lam
     assert np.linalg.norm(A @ x - pair.value * (B @ x)) <= 1e-9 * np.linalg.norm(A @ x)
+
+
+@pytest.mark.parametrize("basis", [0, 1])
+@pytest.mark.parametrize("order", [20, 21, 31, 32, 40, 120])
+def test_fields_of_any_order(ctx, basis, order):
+    """A view filled by hand may hold any order that a byte does; a Mesh's go up to 20."""
+    print(f"[shapes] fields basis={basis} order={order}", flush=True)
+    dom, _ = cases.mixed_refinements()
+    a = {k: v.copy() if isinstance(v, np.ndarray) else v for k, v in dom.arrays().items()}
+    a["bs_i"][::3] = order
+    a["bs_j"][1::4] = order
+    a["orders"][0] = order
+    view, keep = _view_from_arrays(a)
+    sol = np.random.default_rng(order).standard_normal(dom.num_dofs)
+    d = 17
+    rc, ex, ey = oracle.xy_fields(view, basis, (d, d), sol)
+    assert rc == 0
+    gx, gy = np.empty_like(ex), np.empty_like(ey)
+    p = [x.ctypes.data_as(C.POINTER(C.c_double)) for x in (sol, gx, gy)]
+    rc = N.load().fem2d_xy_fields(ctx._h, C.byref(view), basis, d, d, p[0], sol.size, p[1], p[2])
+    assert rc == N.OK, N.last_error()
+    for got, exp in ((gx, ex), (gy, ey)):
+        err = np.abs(got - exp).max() / np.abs(exp).max()
+        assert err <= FIELD_TOL
