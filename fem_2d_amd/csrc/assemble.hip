@@ -253,6 +253,16 @@ struct FillOut {
 
 __device__ __forceinline__ void set_err(int* err, int bits) { atomicOr(err, bits); }
 
+// Whether an error was reported before the block came to look, as one answer for all of
+// its threads: blocks of the same launch report errors too, and a wavefront that left on
+// its own reading would leave the others without what it sets up for the block.
+__device__ __forceinline__ bool block_stops(const int* err) {
+  __shared__ int stop;
+  if (threadIdx.x == 0) stop = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  return stop != 0;
+}
+
 __device__ __forceinline__ int n_groups_of(const Work& w) { return w.n_dofs > 0 ? w.dof_grp[w.n_dofs - 1] : 0; }
 
 // ---------------------------------------------------------------------------
@@ -1813,8 +1823,14 @@ __device__ bool describe_rows(const DevView& v, const Work& w, int g0, bool act,
 // The row groups' records for the streaming fill: headers, source records and
 // column records (the rows' packed specs are written by the DoF-group scan).
 __global__ void __launch_bounds__(kBlock, kDescribeWavesPerSimd) k_describe(DevView v, Work w) {
-  if (*w.err) return;  // an invalid view was detected: nothing below may trust it
   __shared__ DescribeShared shared[kWavesPerBlock];
+  // groups that need a whole wavefront are shared out over the block's wavefronts at
+  // the end: they come in clusters (the edges of one much refined Elem), and four
+  // of them one after another on the wavefront that met them ended the kernel 10 us late
+  constexpr int kList = 128;
+  __shared__ int list[kList], n_list;
+  if (threadIdx.x == 0) n_list = 0;
+  if (block_stops(w.err)) return;  // an invalid view was detected: nothing below may trust it
   const int lane = threadIdx.x % kWave;
   const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   DescribeShared& S = shared[wid];
@@ -1830,13 +1846,6 @@ __global__ void __launch_bounds__(kBlock, kDescribeWavesPerSimd) k_describe(DevV
       describe_group(v, w, g, S.wave, lane);
     return;
   }
-  // groups that need a whole wavefront are shared out over the block's wavefronts at
-  // the end: they come in clusters (the edges of one much refined Elem), and four
-  // of them one after another on the wavefront that met them ended the kernel 10 us late
-  constexpr int kList = 128;
-  __shared__ int list[kList], n_list;
-  if (threadIdx.x == 0) n_list = 0;
-  __syncthreads();
   // static assignment: a shared work counter would serialise on device-scope
   // atomics, which span the XCDs' separate L2 caches
   const int stride = gridDim.x * kWavesPerBlock * kRowsPerWave;

@@ -133,3 +133,35 @@ def test_fields_of_any_order(ctx, basis, order):
     for got, exp in ((gx, ex), (gy, ey)):
         err = np.abs(got - exp).max() / np.abs(exp).max()
         assert err <= FIELD_TOL
+
+
+def _nested_pair_dof(a):
+    """Order-1 arrays with one DoF's specs on an Elem and one of its descendants, by exchanging one
+    spec each of two DoFs: columns of its row group receive more than two contributions."""
+    a = {k: v.copy() if isinstance(v, np.ndarray) else v for k, v in a.items()}
+    elem = np.repeat(np.arange(a["n_elems"]), np.diff(a["bs_offsets"]))
+    specs = a["dof_bs"].reshape(-1, 2)
+    parent = a["parent"]
+    for p, (t0, t1) in enumerate(specs):
+        for q, (t2, t3) in enumerate(specs):
+            if p != q and parent[elem[t3]] == elem[t0] and elem[t2] != elem[t1]:
+                specs[p, 1], specs[q, 1] = t3, t1
+                a["bs_dof"][t3], a["bs_dof"][t1] = p, q
+                return a
+    raise AssertionError("no such pair of DoFs")
+
+
+# 32 row groups (one a wavefront) and 18 389 (four a wavefront)
+@pytest.mark.parametrize("nx,ny,levels", [(4, 2, 2), (64, 32, 3)])
+def test_error_while_describing(ctx, nx, ny, levels):
+    """An error that the describe kernel itself reports, so that its later blocks start after it."""
+    print(f"[shapes] error while describing {nx}x{ny} levels={levels}", flush=True)
+    dom = F.Domain.from_mesh(W.waveguide_64x32_mesh(nx, ny, order=1, levels=levels))
+    view, keep = _view_from_arrays(_nested_pair_dof(dom.arrays()))
+    out = N.GepCsr()
+    rc = N.load().fem2d_galerkin_sample_gep_hcurl(ctx._h, C.byref(view), 0, 0, 1, 8, 8, 0, C.byref(out))
+    assert rc == N.ERR_INVALID_VIEW and "two contributions" in N.last_error(), (rc, N.last_error())
+    gep = F.galerkin_sample_gep_hcurl(dom, (8, 8), F.HierPoly, ctx=ctx)
+    rc, ref = oracle.assemble(dom.view(), basis=F.HierPoly.code, glq=(8, 8), n_threads=8)
+    assert rc == 0
+    assert_gep_matches(gep, ref)
