@@ -2007,7 +2007,7 @@ template <bool kLibInLds, bool kACurlCurl, bool kBCurlCurl, int P>
 __global__ void __launch_bounds__(kFillBlock, kFillWavesPerSimd) k_fill_flat(Work w, LibShape L, FillOut o) {
   using VA = typename Store<P>::A;
   using VB = typename Store<P>::B;
-  if (*w.err) return;
+  if (block_stops(w.err)) return;  // so that every wavefront is there to ask for tickets and to answer
   __shared__ FillShared shared[kFillBlock / kWave];
   __shared__ FillRounds rounds;
   // the block's copy of the Gram library (when it fits)

@@ -165,3 +165,20 @@ def test_error_while_describing(ctx, nx, ny, levels):
     rc, ref = oracle.assemble(dom.view(), basis=F.HierPoly.code, glq=(8, 8), n_threads=8)
     assert rc == 0
     assert_gep_matches(gep, ref)
+
+
+@pytest.mark.parametrize("precision", [F.FP64, F.FP32])
+def test_many_rounds_of_chunks(ctx, precision):
+    """25.7 M entries in chunks of 64: about 98 rounds a block, past the 64 tickets that the fill's ring
+    keeps, against the few rounds that the automatic size makes."""
+    print(f"[shapes] many rounds precision={precision}", flush=True)
+    w = W.waveguide_64x32()
+    dd = F.DeviceDomain(w.domain, ctx)
+    ref = dd.download(dd.assemble(w.glq, F.HierPoly, precision=precision))
+    ctx.set_fill_chunk(64)
+    try:
+        got = dd.download(dd.assemble(w.glq, F.HierPoly, precision=precision))
+    finally:
+        ctx.set_fill_chunk(0)
+    assert ref.nnz == 25_704_606
+    _same_bits(got, ref)
