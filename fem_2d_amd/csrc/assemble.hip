@@ -2488,7 +2488,7 @@ __device__ bool build_group(const DevView& v, const Work& w, int g, GroupShared&
 }
 
 __global__ void __launch_bounds__(kBlock) k_count_large(DevView v, Work w) {
-  if (*w.err) return;  // an invalid view was detected: nothing below may trust it
+  if (block_stops(w.err)) return;  // an invalid view was detected: nothing below may trust it
   extern __shared__ unsigned char smem[];
   GroupShared& S = *reinterpret_cast<GroupShared*>(smem);
   const int n_large = *w.n_large;
@@ -2516,7 +2516,7 @@ __global__ void __launch_bounds__(kBlock) k_count_large(DevView v, Work w) {
 // spec list before it is used; a violation sets kErrView and the entry is
 // skipped.
 __global__ void __launch_bounds__(kBlock) k_fill_large(DevView v, Work w, LibShape L, FillOut o) {
-  if (*w.err) return;  // an invalid view was detected: nothing below may trust it
+  if (block_stops(w.err)) return;  // an invalid view was detected: nothing below may trust it
   // the host grows the buffers and runs the assembly again (as k_fill_flat)
   if (w.row_ptr[w.n_dofs] > o.capacity) return;
   extern __shared__ unsigned char smem[];

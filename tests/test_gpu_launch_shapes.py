@@ -141,10 +141,15 @@ def _nested_pair_dof(a):
     a = {k: v.copy() if isinstance(v, np.ndarray) else v for k, v in a.items()}
     elem = np.repeat(np.arange(a["n_elems"]), np.diff(a["bs_offsets"]))
     specs = a["dof_bs"].reshape(-1, 2)
-    parent = a["parent"]
+
+    def below(e, top):
+        while e >= 0 and e != top:
+            e = a["parent"][e]
+        return e == top
+
     for p, (t0, t1) in enumerate(specs):
         for q, (t2, t3) in enumerate(specs):
-            if p != q and parent[elem[t3]] == elem[t0] and elem[t2] != elem[t1]:
+            if p != q and below(elem[t3], elem[t0]) and elem[t3] != elem[t0] and elem[t2] != elem[t1]:
                 specs[p, 1], specs[q, 1] = t3, t1
                 a["bs_dof"][t3], a["bs_dof"][t1] = p, q
                 return a
@@ -182,3 +187,25 @@ def test_many_rounds_of_chunks(ctx, precision):
         ctx.set_fill_chunk(0)
     assert ref.nnz == 25_704_606
     _same_bits(got, ref)
+
+
+def test_error_while_counting(ctx):
+    """An error that the block path's counting kernel reports: an edge between an Elem with 84
+    descendants and its neighbour, with one DoF's second spec moved into a descendant."""
+    print("[shapes] error while counting", flush=True)
+    mesh = F.Mesh.rect_grid(2, 1, 0.0, 1.0, 0.0, 0.5)
+    mesh.set_global_expansion_orders(F.Orders(1, 1))
+    leaves = [0]
+    for _ in range(3):
+        mesh.execute_h_refinements([(e, F.HRef.t()) for e in leaves])
+        leaves = [c for e in leaves for c in mesh.elem(e).child_ids()]
+    dom = F.Domain.from_mesh(mesh)
+    gep = F.galerkin_sample_gep_hcurl(dom, (8, 8), F.HierPoly, ctx=ctx)
+    assert ctx.last_timing()["n_large"] > 0
+    rc, ref = oracle.assemble(dom.view(), basis=F.HierPoly.code, glq=(8, 8), n_threads=8)
+    assert rc == 0
+    assert_gep_matches(gep, ref)
+    view, keep = _view_from_arrays(_nested_pair_dof(dom.arrays()))
+    out = N.GepCsr()
+    rc = N.load().fem2d_galerkin_sample_gep_hcurl(ctx._h, C.byref(view), 0, 0, 1, 8, 8, 0, C.byref(out))
+    assert rc == N.ERR_INVALID_VIEW and "two contributions" in N.last_error(), (rc, N.last_error())
