@@ -202,6 +202,8 @@ struct Work {
   const int* range_map;
   int range_map_v;
   int* err;
+  long long* status;  // the call's status block (null while a Domain is prepared): nnz, error bits,
+                      // block-path groups, row groups
   int* n_large;       // row groups handled by the block path
   int* ticket;        // chunk rounds that the streaming fill's blocks have taken
   int* large_list;
@@ -251,7 +253,13 @@ struct FillOut {
   int precision;  // fem2d_precision
 };
 
-__device__ __forceinline__ void set_err(int* err, int bits) { atomicOr(err, bits); }
+// Reports an error to the kernels that follow and to the call. The layout writes the
+// error word into the status block; what a later kernel reports goes there directly
+// (the status of any one of them will do).
+__device__ __forceinline__ void set_err(const Work& w, int bits) {
+  atomicOr(w.err, bits);
+  if (w.status) __hip_atomic_store(w.status + 1, (long long)bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Whether an error was reported before the block came to look, as one answer for all of
 // its threads: blocks of the same launch report errors too, and a wavefront that left on
@@ -417,7 +425,7 @@ __device__ __forceinline__ void block_coefs(const Work& w, int P, int Q, bool lo
     ru = rel_range_id(w, dp, dq, 0);
     rv = rel_range_id(w, dp, dq, 1);
     if (ru < 0 || rv < 0) {  // a position the upload did not see: the view is inconsistent
-      set_err(w.err, kErrView);
+      set_err(w, kErrView);
       ru = rv = 0;
     }
     su = ldexp(1.0, -(dq.x - dp.x));
@@ -543,7 +551,7 @@ __device__ __forceinline__ void elem_prep_body(const DevView& v, const Work& w, 
   while (v.parent[x] >= 0) {
     const int p = v.parent[x];
     if (p >= v.n_elems || p == x || depth >= kMaxDepth) {
-      set_err(w.err, p >= v.n_elems || p == x ? kErrView : kErrDepth);
+      set_err(w, p >= v.n_elems || p == x ? kErrView : kErrDepth);
       return;
     }
     locs[depth++] = v.loc[x];
@@ -558,7 +566,7 @@ __device__ __forceinline__ void elem_prep_body(const DevView& v, const Work& w, 
     const double mu = (u0 + u1) / 2.0, mv = (v0 + v1) / 2.0;
     const int l = locs[t];
     if (l > FEM2D_LOC_N) {
-      set_err(w.err, kErrView);
+      set_err(w, kErrView);
       return;
     }
     const bool split_u = l <= FEM2D_LOC_E;  // SW, SE, NW, NE, W, E
@@ -628,7 +636,7 @@ __device__ __forceinline__ void spec_body(const DevView& v, const Work& w, long 
       // H(curl) specs are U or V directed with orders inside the Gram library
       if (d < 0 || d >= v.n_dofs || v.bs_dir[t] > FEM2D_DIR_V || v.bs_i[t] >= v.p1 || v.bs_j[t] >= v.p1 ||
           (v.dof_bs[2LL * d] != t && v.dof_bs[2LL * d + 1] != t))
-        set_err(w.err, kErrView);
+        set_err(w, kErrView);
     }
   }
 }
@@ -641,7 +649,7 @@ __device__ __forceinline__ void dof_check_body(const DevView& v, const Work& w, 
   const int ta = v.dof_bs[2 * d], tb = v.dof_bs[2 * d + 1];
   const bool ok_a = ta >= 0 && ta < v.n_bs && v.bs_dof[ta] == d;
   const bool ok_b = tb == -1 || (tb >= 0 && tb < v.n_bs && tb != ta && v.bs_dof[tb] == d);
-  if (!ok_a || !ok_b) set_err(w.err, kErrView);
+  if (!ok_a || !ok_b) set_err(w, kErrView);
 }
 
 // A DoF's signature: the Elems of its specs in increasing order and the specs
@@ -830,12 +838,12 @@ struct DofGroupScan {
     const int k = int(pos & kPosIndex);
     const bool start = (pos & kPosPrevAdj) == 0u || first;
     const bool end = (pos & kPosNextAdj) == 0u || last;
-    if ((start && !first) || (end && !last)) set_err(w.err, kErrView);  // a run that is not a whole group
+    if ((start && !first) || (end && !last)) set_err(w, kErrView);  // a run that is not a whole group
     w.spec_run[t] = make_int2(start ? g : -1, k);
   }
   __device__ void store(long long d, long long excl, const Item& it) const {
     const int e1 = it.sig.x, e2 = it.sig.z;
-    if (e1 < 0 || (e2 >= 0 && e2 == e1)) set_err(w.err, kErrView);  // no spec, or two on one Elem
+    if (e1 < 0 || (e2 >= 0 && e2 == e1)) set_err(w, kErrView);  // no spec, or two on one Elem
     const int g1 = int(excl + it.n);  // group id + 1
     w.dof_grp[d] = g1;
     if (it.n) {
@@ -1158,8 +1166,8 @@ __global__ void __launch_bounds__(kBlock) k_scan_apply(long long n, Op op, const
 // block-path groups, row groups). Without tile_sum (few groups) every block sums the
 // groups before its own, and `parts` blocks share a tile's chunks (94 groups of 3 700
 // entries: 13.8 us with one block, 5.2 with eight).
-__global__ void __launch_bounds__(kBlock) k_layout(Work w, long long n_items, const long long* tile_sum, int parts,
-                                                   long long* status) {
+__global__ void __launch_bounds__(kBlock) k_layout(Work w, long long n_items, const long long* tile_sum,
+                                                   int parts) {
   __shared__ long long s_wave[kWavesPerBlock], s_pre[kWavesPerBlock], s_all[kWavesPerBlock];
   const GroupScan op{w};
   const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
@@ -1210,10 +1218,10 @@ __global__ void __launch_bounds__(kBlock) k_layout(Work w, long long n_items, co
     if (g < n_items && part == 0) w.seg_start[g] = start;
     if (g == n_items - 1 && part == 0) {
       w.row_ptr[w.n_dofs] = start;
-      status[0] = start;
-      status[1] = *w.err;
-      status[2] = *w.n_large;
-      status[3] = n_groups;
+      w.status[0] = start;
+      w.status[1] = *w.err;
+      w.status[2] = *w.n_large;
+      w.status[3] = n_groups;
     }
     const long long C = fill_chunk(w, nnz);
     // chunks [c, c1) start in the segment
@@ -1444,7 +1452,7 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
   }
   if (__ballot(bad != 0)) {
     if (__ballot((bad & 2) != 0)) {
-      if (lane == 0) set_err(w.err, kErrContrib);
+      if (lane == 0) set_err(w, kErrContrib);
       return 2;
     }
     return 1;
@@ -1470,7 +1478,7 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
   }
   wave_sync();
   if (S.u_self < 0) {
-    if (lane == 0) set_err(w.err, kErrView);
+    if (lane == 0) set_err(w, kErrView);
     return 2;
   }
   if (S.total - S.u_self > kWC || ld_const(w.g_start, g + 1) - gs_self > kWRows) return 1;
@@ -1726,7 +1734,7 @@ __device__ bool describe_rows(const DevView& v, const Work& w, int g0, bool act,
     wave_sync();
   }
   if (row_ballot(bad, row)) {
-    if (bad) set_err(w.err, kErrContrib);
+    if (bad) set_err(w, kErrContrib);
     act = false;
   }
   // columns before each distinct group; the group itself among them
@@ -1748,7 +1756,7 @@ __device__ bool describe_rows(const DevView& v, const Work& w, int g0, bool act,
   wave_sync();
   const int self = S.self;
   if (act && self < 0) {  // the group is not among its own candidates
-    if (sl == 0) set_err(w.err, kErrView);
+    if (sl == 0) set_err(w, kErrView);
     act = false;
   }
   const int u_self = act ? S.u_self : 0;
@@ -1836,7 +1844,7 @@ __global__ void __launch_bounds__(kBlock, kDescribeWavesPerSimd) k_describe(DevV
   DescribeShared& S = shared[wid];
   const int n_groups = n_groups_of(w);
   // more row groups than the view's DoF signatures give have no room for records
-  if (n_groups > w.meta_cap && blockIdx.x == 0 && threadIdx.x == 0) set_err(w.err, kErrView);
+  if (n_groups > w.meta_cap && blockIdx.x == 0 && threadIdx.x == 0) set_err(w, kErrView);
   const int n = min(n_groups, w.meta_cap);
   // few groups: one a wavefront. Four share one chain of dependent loads, which is a
   // gain once there are more groups than wavefronts to start them (17 080 groups
@@ -2124,7 +2132,7 @@ __global__ void __launch_bounds__(kFillBlock, kFillWavesPerSimd) k_fill_flat(Wor
       if (over) limit = min(limit, __builtin_amdgcn_readlane(s, __builtin_ctzll(over)));
       if (limit < len && (limit & ~(kWave - 1)) > pos) limit &= ~(kWave - 1);
       if (limit <= pos) {  // the first row holds entry pos: the layout disagrees with itself
-        if (lane == 0) set_err(w.err, kErrView);
+        if (lane == 0) set_err(w, kErrView);
         break;
       }
       const bool in = lead && valid && s < limit;
@@ -2314,7 +2322,7 @@ __device__ bool build_group(const DevView& v, const Work& w, int g, GroupShared&
   const int tid = threadIdx.x;
   const int n = gather_sources(w, g, kMaxSrc, S.src_x, S.src_info, tid, blockDim.x);
   if (n > kMaxSrc) {  // block-uniform
-    if (tid == 0) set_err(w.err, kErrSize);
+    if (tid == 0) set_err(w, kErrSize);
     return false;
   }
   __syncthreads();
@@ -2330,7 +2338,7 @@ __device__ bool build_group(const DevView& v, const Work& w, int g, GroupShared&
   int n_raw = 0;
   const int first_raw = block_excl_scan(cnt, S.wave_sum, &n_raw);
   if (n_raw > kMaxRaw) {  // block-uniform
-    if (tid == 0) set_err(w.err, kErrSize);
+    if (tid == 0) set_err(w, kErrSize);
     return false;
   }
   if (tid < n) {
@@ -2410,7 +2418,7 @@ __device__ bool build_group(const DevView& v, const Work& w, int g, GroupShared&
   int nd = 0;
   const int first = block_excl_scan(n_new, S.wave_sum, &nd);
   if (nd > kMaxDist) {  // block-uniform
-    if (tid == 0) set_err(w.err, kErrSize);
+    if (tid == 0) set_err(w, kErrSize);
     return false;
   }
   {
@@ -2481,7 +2489,7 @@ __device__ bool build_group(const DevView& v, const Work& w, int g, GroupShared&
   const int fail = S.fail;
   __syncthreads();
   if (fail) {
-    if (tid == 0) set_err(w.err, fail == 2 ? kErrContrib : (fail == 3 ? kErrView : kErrSize));
+    if (tid == 0) set_err(w, fail == 2 ? kErrContrib : (fail == 3 ? kErrView : kErrSize));
     return false;
   }
   return true;
@@ -2496,7 +2504,7 @@ __global__ void __launch_bounds__(kBlock) k_count_large(DevView v, Work w) {
     const int g = w.large_list[i];
     const int r0 = w.g_start[g], r1 = w.g_start[g + 1];
     if (r1 - r0 > kMaxRows) {
-      if (threadIdx.x == 0) set_err(w.err, kErrSize);
+      if (threadIdx.x == 0) set_err(w, kErrSize);
       continue;
     }
     if (!build_group<false>(v, w, g, S)) continue;
@@ -2534,7 +2542,7 @@ __global__ void __launch_bounds__(kBlock) k_fill_large(DevView v, Work w, LibSha
     const int T = S.total - S.u_self;  // candidate columns of the group's first row
     // the segment holds rows of T, T - 1, ... entries (block-uniform check)
     if (seg_len != (long long)nrows * T - (long long)nrows * (nrows - 1) / 2 || nrows > T) {
-      if (threadIdx.x == 0) set_err(w.err, kErrView);
+      if (threadIdx.x == 0) set_err(w, kErrView);
       __syncthreads();
       continue;
     }
@@ -2559,7 +2567,7 @@ __global__ void __launch_bounds__(kBlock) k_fill_large(DevView v, Work w, LibSha
       }
       const int u = S.u_self + lo + (p - S.row_rel[lo]);
       if (u < S.u_self || u >= S.total) {  // outside the candidate set: the layout disagrees with it
-        set_err(w.err, kErrView);
+        set_err(w, kErrView);
         continue;
       }
       int a = 0, b = n_dist;
@@ -2594,7 +2602,7 @@ __global__ void __launch_bounds__(kBlock) k_fill_large(DevView v, Work w, LibSha
         l2_sum += l2;
       }
       if (!ok) {
-        set_err(w.err, kErrView);
+        set_err(w, kErrView);
         continue;
       }
       write_entry(o, seg0 + p, c, cc_sum, l2_sum);
@@ -3282,10 +3290,10 @@ void ensure_glq(fem2d_ctx* ctx, int nu, int nv) {
 }
 
 // Part (a): preparation and symbolic phase, ending with the CSR layout and the
-// status block (nnz, error bits, block-path groups, row groups) at status.
+// status block (Work::status).
 // With fine_events, events between the stages time them and the describe
 // kernel.
-int launch_prep(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, long long* status, bool fine_events) {
+int launch_prep(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, bool fine_events) {
   const Work& w = a.w;
   const DevView& v = a.v;
   const int ne = v.n_elems;
@@ -3324,7 +3332,7 @@ int launch_prep(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, long long* st
   const int parts = two_pass ? 1 : 8;
   if (two_pass) k_scan_reduce<<<scan_grid(a.tiles_grp), kBlock, 0, st>>>(a.n_grp_items, GroupScan{w}, a.ts_grp);
   k_layout<<<scan_grid(a.tiles_grp) * unsigned(parts), kBlock, 0, st>>>(w, a.n_grp_items,
-                                                                        two_pass ? a.ts_grp : nullptr, parts, status);
+                                                                        two_pass ? a.ts_grp : nullptr, parts);
   HIP_TRY_AT(hipGetLastError(), "after the CSR layout scan");
   if (fine_events) HIP_TRY(hipEventRecord(ctx->ev[2], st));
   return FEM2D_OK;
@@ -3759,6 +3767,7 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
   if (rc) return rc;
   Work& w = a.w;
   set_chunk(ctx, a, precision);
+  w.status = ctx->d_status;
   const bool run_large = a.run_large;
   hipStream_t st = ctx->stream;
   ensure_glq(ctx, nu, nv);
@@ -3810,7 +3819,7 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
       const GraphKey key{dd->serial, basis,     ai,       bi, nu, nv, o.capacity, g_alloc_generation.load(),
                          run_large,  precision, w.chunk};
       auto whole = [&]() -> int {
-        int prc = launch_prep(ctx, st, a, ctx->d_status, false);
+        int prc = launch_prep(ctx, st, a, false);
         if (prc != FEM2D_OK) return prc;
         // the block-path fill writes segments of its own, from row pointers the
         // layout scan wrote: a branch beside the streaming fill (a branch
@@ -3847,7 +3856,7 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
       fine_timing = false;
     } else {
       HIP_TRY(hipEventRecord(ctx->ev[0], st));
-      if ((rc = launch_prep(ctx, st, a, ctx->d_status, true))) return rc;
+      if ((rc = launch_prep(ctx, st, a, true))) return rc;
       HIP_TRY(hipEventRecord(ctx->ev[6], st));
       if (fill && (rc = launch_stream_fill(ctx, st, a, o))) return rc;
       HIP_TRY(hipEventRecord(ctx->ev[7], st));
@@ -3943,6 +3952,7 @@ int fem2d_assemble_device_noalloc(fem2d_ctx* ctx, const fem2d_device_domain* dd,
   Work& w = a.w;
   w.row_ptr = row_ptr;
   set_chunk(ctx, a, precision);
+  w.status = ctx->d_status;
   // the table of first rows comes last and takes what is left where that is less
   // than it would like (larger chunks then)
   const size_t at = (used + 255) & ~size_t(255);
@@ -3964,7 +3974,7 @@ int fem2d_assemble_device_noalloc(fem2d_ctx* ctx, const fem2d_device_domain* dd,
   // kernel by kernel on the context's stream: k_gram's clearing blocks reset every counter
   // and flag the kernels accumulate into, so the array's earlier contents do
   // not matter
-  if ((rc = launch_prep(ctx, st, a, ctx->d_status, false))) return rc;
+  if ((rc = launch_prep(ctx, st, a, false))) return rc;
   if (capacity > 0 && (rc = launch_stream_fill(ctx, st, a, o))) return rc;
   if (capacity > 0 && a.run_large && (rc = launch_large_fill(ctx, st, a, o))) return rc;
   HIP_TRY(hipStreamSynchronize(st));
