@@ -56,6 +56,7 @@
 #include "host/parallel.hpp"
 #include "fp32r.hpp"
 #include "domain_build.hpp"
+#include "graph_rule.hpp"
 #include "pinned_staging.hpp"
 
 namespace {
@@ -2804,22 +2805,6 @@ struct DevBuf {
   size_t bytes = 0;
 };
 
-// what a recorded assembly graph depends on besides its buffers
-struct GraphKey {
-  unsigned long long domain = 0;
-  int basis = -1, ai = -1, bi = -1, nu = 0, nv = 0;
-  long long capacity = -1;
-  unsigned long long alloc_generation = 0;
-  bool run_large = true;
-  int precision = -1;
-  int chunk = 0;
-  bool operator==(const GraphKey& o) const {
-    return domain == o.domain && basis == o.basis && ai == o.ai && bi == o.bi && nu == o.nu && nv == o.nv &&
-           capacity == o.capacity && alloc_generation == o.alloc_generation && run_large == o.run_large &&
-           precision == o.precision && chunk == o.chunk;
-  }
-};
-
 std::atomic<unsigned long long> g_domain_serial{0};
 
 }  // namespace
@@ -2894,9 +2879,8 @@ struct fem2d_ctx {
   int fill_grid[kPrecisions][2] = {};  // resident blocks of the fill per precision and FillPlace
   bool use_graphs = true;
   int fill_chunk = 0;  // fill chunk size forced for every assembly (0: fill_chunk_of's)
-  hipGraphExec_t graph_exec[1] = {nullptr};  // the last recorded assembly
-  GraphKey graph_key;
-  GraphKey last_key;  // of the latest assembly: only the second in a row of a key is recorded
+  hipGraphExec_t graph_exec = nullptr;  // the last recorded assembly
+  fem2d::GraphRule graph_rule;
   void* solver = nullptr;  // eigensolver handle, made by the first solve
   // generation of the latest assembly whose outputs the buffers hold (0: none)
   unsigned long long out_generation = 0;
@@ -3543,8 +3527,7 @@ void fem2d_ctx_destroy(fem2d_ctx* ctx) {
     if (b.p) (void)hipFree(b.p);
   for (DevBuf* b : {&ctx->out_col, &ctx->out_a, &ctx->out_b, &ctx->out_r})
     if (b->p) (void)hipFree(b->p);
-  for (auto& g : ctx->graph_exec)
-    if (g) (void)hipGraphExecDestroy(g);
+  if (ctx->graph_exec) (void)hipGraphExecDestroy(ctx->graph_exec);
   for (auto& e : ctx->ev)
     if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : {ctx->fork_ev, ctx->join_ev})
@@ -3775,14 +3758,14 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
   // The assembly in three parts: (a) preparation and symbolic phase, ending
   // with the CSR layout and the status block, (b) the streaming fill, (c) the
   // block-path fill (only for Domains with large row groups). With graphs the
-  // three are recorded as one graph the second time in a row that they come with the same
-  // Domain, options and buffers, replayed while these stay, and timed end to end; kernel by kernel,
-  // events between the stages also time the stages and the describe and fill
+  // three are launched, recorded as one graph or replayed (GraphRule), and timed end to end;
+  // kernel by kernel, events between the stages also time the stages and the describe and fill
   // kernels on their own.
-  // record the work of parts() into ctx->graph_exec[i]
-  auto record = [&](int i, const std::function<int()>& part) -> int {
-    if (ctx->graph_exec[i]) (void)hipGraphExecDestroy(ctx->graph_exec[i]);
-    ctx->graph_exec[i] = nullptr;
+  // record the work of part() into ctx->graph_exec
+  auto record = [&](const std::function<int()>& part) -> int {
+    ctx->graph_rule.forget();
+    if (ctx->graph_exec) (void)hipGraphExecDestroy(ctx->graph_exec);
+    ctx->graph_exec = nullptr;
     (void)hipGetLastError();  // no stale error is reported as a recording failure
     HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     const int erc = part();
@@ -3792,10 +3775,10 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
       if (graph) (void)hipGraphDestroy(graph);
       return erc != FEM2D_OK ? erc : hip_fail(ec, "hipStreamEndCapture");
     }
-    const hipError_t ei = hipGraphInstantiate(&ctx->graph_exec[i], graph, nullptr, nullptr, 0);
+    const hipError_t ei = hipGraphInstantiate(&ctx->graph_exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     if (ei != hipSuccess) {
-      ctx->graph_exec[i] = nullptr;
+      ctx->graph_exec = nullptr;
       return hip_fail(ei, "hipGraphInstantiate");
     }
     return FEM2D_OK;
@@ -3816,8 +3799,8 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
     const bool fill = o.capacity > 0;
     const bool tail = fill && run_large;  // part (c) has work
     if (ctx->use_graphs) {
-      const GraphKey key{dd->serial, basis,     ai,       bi, nu, nv, o.capacity, g_alloc_generation.load(),
-                         run_large,  precision, w.chunk};
+      const fem2d::GraphKey key{dd->serial, basis, ai, bi, nu, nv, o.capacity, g_alloc_generation.load(),
+                                run_large, precision, w.chunk};
       auto whole = [&]() -> int {
         int prc = launch_prep(ctx, st, a, false);
         if (prc != FEM2D_OK) return prc;
@@ -3834,24 +3817,16 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
         if (tail) HIP_TRY(hipStreamWaitEvent(st, ctx->join_ev, 0));
         return prc;
       };
-      const bool recorded = ctx->graph_exec[0] && key == ctx->graph_key;
-      if (!recorded && key == ctx->last_key) {
-        ctx->graph_key = GraphKey{};
-        if ((rc = record(0, whole))) return rc;
-        ctx->graph_key = key;
+      const auto step = ctx->graph_rule.step(key);
+      if (step == fem2d::GraphRule::kRecord) {
+        if ((rc = record(whole))) return rc;
+        ctx->graph_rule.made(key);
       }
       // only the end points of the whole assembly are timed
       HIP_TRY(hipEventRecord(ctx->ev[0], st));
-      if (key == ctx->graph_key) {
-        HIP_TRY(hipGraphLaunch(ctx->graph_exec[0], st));
-      } else {
-        // not the same Domain, options and buffers as the assembly before: a Domain of
-        // an adaptive loop or of a drop-in call is assembled only once, and a
-        // recording costs more than the launches it saves (the assembly of a new
-        // hp-irregular 32 x 16 Domain 310 us recorded and replayed, 177 launched)
-        if ((rc = whole())) return rc;
-      }
-      ctx->last_key = key;
+      if (step != fem2d::GraphRule::kLaunch) HIP_TRY(hipGraphLaunch(ctx->graph_exec, st));
+      else if ((rc = whole())) return rc;
+      ctx->graph_rule.came(key);
       HIP_TRY(hipEventRecord(ctx->ev[3], st));
       fine_timing = false;
     } else {
@@ -3892,6 +3867,7 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
     return fem2d_assemble_device(ctx, dd, basis, ai, bi, glq_u, glq_v, precision, out);
   }
   dd->large_state = n_large > 0 ? 1 : 0;
+  if (ctx->use_graphs) ctx->graph_rule.learned(n_large > 0);
   ctx->timing.fill_chunk = w.chunk ? w.chunk : fill_chunk_of(nnz, w.chunk_cap, w.fill_waves, w.chunk_max);
   ctx->timing.fill_lib_lds = fill_place(a.lib_n);
 

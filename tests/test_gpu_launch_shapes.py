@@ -209,3 +209,23 @@ def test_error_while_counting(ctx):
     out = N.GepCsr()
     rc = N.load().fem2d_galerkin_sample_gep_hcurl(ctx._h, C.byref(view), 0, 0, 1, 8, 8, 0, C.byref(out))
     assert rc == N.ERR_INVALID_VIEW and "two contributions" in N.last_error(), (rc, N.last_error())
+
+
+@pytest.mark.parametrize("precision", [F.FP64, F.FP32, F.FP32R])
+@pytest.mark.parametrize("make", [cases.small_hp_irregular, W.waveguide_64x32])
+def test_replays_in_every_precision(precision, make):
+    """An assembly launched, recorded and replayed twice, with and without block-path row groups, each
+    with the bits of a context that launches kernel by kernel and that works in between."""
+    print(f"[shapes] replays precision={precision} {make.__name__}", flush=True)
+    w = make()
+    dom, glq = w if isinstance(w, tuple) else (w.domain, w.glq)
+    c, eager = F.Context(0), F.Context(0)
+    eager.set_graphs(False)
+    dd, ed = F.DeviceDomain(dom, c), F.DeviceDomain(dom, eager)
+    ref = ed.download(ed.assemble(glq, F.KOLShapeFn, precision=precision))
+    for _ in range(4):
+        _same_bits(dd.download(dd.assemble(glq, F.KOLShapeFn, precision=precision)), ref)
+        ed.assemble(glq, F.HierPoly, precision=precision)
+        eager.synchronize()
+    c.close()
+    eager.close()
