@@ -6,6 +6,7 @@ _compare.RTOL of the oracle, fields within 1e-13 of the largest (as in the field
 forced chunks and graph replays give the same bits."""
 
 import ctypes as C
+import re
 
 import numpy as np
 import pytest
@@ -18,6 +19,7 @@ from _compare import assert_gep_matches
 from fem_2d_amd import _native as N
 from fem_2d_amd import workloads as W
 from test_gpu_parity import _view_from_arrays
+from test_zz_no_alloc import DeviceArrays, check_same, noalloc
 
 pytestmark = pytest.mark.gpu
 
@@ -229,3 +231,42 @@ def test_replays_in_every_precision(precision, make):
         eager.synchronize()
     c.close()
     eager.close()
+
+
+def test_first_row_table_short_of_scratch():
+    """A Domain that leaves the no-allocation entry point less of its scratch array than the table of
+    the chunks' first rows would take: larger chunks, and the same bits. Orders of 5 instead of 4 on
+    more and more Elems use the array up; an absurd capacity has the call say what it needs."""
+    print("[shapes] first-row table short of scratch", flush=True)
+    ctx = F.Context(0)
+    nothing = DeviceArrays(ctx, 100_000, 0, 8)
+    absurd = 4096 << 25  # a table of 2^25 + 1 words at least
+
+    def domain(k):
+        mesh = W.waveguide_64x32_mesh(76, 43, order=4, levels=0)
+        mesh.set_expansion_on_elems(range(k), F.Orders(5, 5))
+        return F.Domain.from_mesh(mesh)
+
+    def words_left(dom):
+        rc, _ = noalloc(ctx, F.DeviceDomain(dom, ctx), (8, 8), F.HierPoly, F.FP64, nothing, absurd)
+        assert rc == N.ERR_UNSUPPORTED, (rc, N.last_error())
+        need, size = map(int, re.search(r"needs (\d+) bytes.* has (\d+) ", N.last_error()).groups())
+        return (size - (need - 4 * (absurd // 4096 + 1))) // 4
+
+    k, end = 0, 76 * 43  # more than 2 000 words are left at k, fewer at the end
+    assert words_left(domain(k)) > 2000 >= words_left(domain(end))
+    while end - k > 1:
+        mid = (k + end) // 2
+        if words_left(domain(mid)) > 2000:
+            k = mid
+        else:
+            end = mid
+    dom = domain(k)
+    dd = F.DeviceDomain(dom, ctx)
+    nnz = dd.assemble((8, 8), F.HierPoly).nnz
+    chunk = ctx.last_timing()["fill_chunk"]
+    assert nnz // 4096 + 1 < words_left(dom) < nnz // chunk
+    for precision in (F.FP64, F.FP32):
+        check_same(ctx, dom, (8, 8), F.HierPoly, precision).free()
+    nothing.free()
+    ctx.close()
