@@ -208,7 +208,6 @@ struct Work {
   int* n_large;       // row groups handled by the block path
   int* ticket;        // chunk rounds that the streaming fill's blocks have taken
   int* large_list;
-  unsigned char* is_large;
   // per row group, fixed-stride records written by the describe kernel and
   // streamed by the fill kernel (groups of the block path have T = -1)
   int4* meta_hdr;      // [G] T (first row's length), rows, sources, first row
@@ -1321,7 +1320,7 @@ __device__ __forceinline__ int wave_incl_scan(int x) {
 // Per-wave LDS of the candidate-set build by a whole wavefront
 struct WaveShared {
   int src_x[kWS];
-  int src_info[kWS];  // k | rel << 1 | ru << 3 | rv << 17
+  int src_info[kWS];  // k | rel << 1
   int src_bs[kWS];    // first basis spec of each source (bs_offsets)
   int src_m0[kWS];    // first membership of each source
   int raw_base[kWS];  // first raw candidate of each source
@@ -1352,9 +1351,8 @@ __device__ __forceinline__ void write_source(const Work& w, double* out, const d
 
 // Builds row group g's candidate set in this wave's LDS slice. Returns 0 when
 // built and inside the wave path's limits, 1 when the group needs the block
-// path, 2 on an invalid domain (error flag set). With coef non-null the
-// per-source prefactors are written there (kCoef doubles per source) and the
-// source infos gain their dyadic range ids.
+// path, 2 on an invalid domain (error flag set). The source records (kCoef
+// doubles each) are written to the group's slots at coef.
 __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S, int lane, double* coef) {
   const int n_src = gather_sources(w, g, kWS, S.src_x, S.src_info, lane, kWave);
   if (n_src > kWS) return 1;
@@ -1391,18 +1389,15 @@ __device__ int wave_build(const DevView& v, const Work& w, int g, WaveShared& S,
     S.raw_meta[r] = a | (w.mem_bsoff[m] << 8);
   }
   if (lane < n_src) {
-    if (coef) {
-      const int info = S.src_info[lane];
-      const int k = info & 1, rel = (info >> 1) & 3;
-      const int E = k == 0 ? w.g_e1[g] : w.g_e2[g];
-      const int P = rel == kAnc ? X : E;
-      const int Q = rel == kAnc ? E : X;
-      int ru, rv;
-      double cA[4], cB[2];
-      block_coefs(w, P, Q, rel == kLocal, cA, cB, ru, rv);
-      write_source(w, coef + (src_slot(g, n_src) + lane) * kCoef, cA, cB, ru, rv, rel == kAnc);
-      S.src_info[lane] = k | (rel << 1) | (ru << 3) | (rv << 17);
-    }
+    const int info = S.src_info[lane];
+    const int k = info & 1, rel = (info >> 1) & 3;
+    const int E = k == 0 ? w.g_e1[g] : w.g_e2[g];
+    const int P = rel == kAnc ? X : E;
+    const int Q = rel == kAnc ? E : X;
+    int ru, rv;
+    double cA[4], cB[2];
+    block_coefs(w, P, Q, rel == kLocal, cA, cB, ru, rv);
+    write_source(w, coef + (src_slot(g, n_src) + lane) * kCoef, cA, cB, ru, rv, rel == kAnc);
   }
   wave_sync();  // every raw key is in LDS
   // rank sort by (row group, gather order): the keys are distinct (they carry
@@ -1532,7 +1527,6 @@ __device__ void describe_group(const DevView& v, const Work& w, int g, WaveShare
   const int nrows = r1 - r0;
   if (st == 1) {
     if (lane == 0) {
-      w.is_large[g] = 1;
       w.large_list[atomicAdd(w.n_large, 1)] = g;
       w.meta_hdr[g] = make_int4(-1, nrows, 0, 0);
     }
@@ -1540,7 +1534,6 @@ __device__ void describe_group(const DevView& v, const Work& w, int g, WaveShare
     const int u_self = S.u_self, n_dist = S.n_dist, n_src = S.n_src;  // set by wave_build
     const int T = S.total - u_self;
     if (lane == 0) {
-      w.is_large[g] = 0;
       w.meta_hdr[g] = make_int4(T, nrows, n_src, r0);
     }
     for (int t = lane; t < T; t += kWave) {
@@ -1767,7 +1760,6 @@ __device__ bool describe_rows(const DevView& v, const Work& w, int g0, bool act,
     act = false;
   }
   if (act && sl == 0) {
-    w.is_large[g] = 0;
     w.meta_hdr[g] = make_int4(T, nrows, n_src, r0);
   }
   // the groups' first columns as a bitmap, so that a column finds its group by counting
@@ -3214,7 +3206,7 @@ int bind_work(const fem2d_device_domain* dd, int nu, int nv, int basis, Bind&& b
       (rc = bind(k++, N1, &w.dof_grp)) || (rc = bind(k++, N1, &w.g_start)) || (rc = bind(k++, N1, &w.g_e1)) ||
       (rc = bind(k++, N1, &w.g_e2)) || (rc = bind(k++, B1, &w.mem_idx)) || (rc = bind(k++, B1, &w.mem_group)) ||
       (rc = bind(k++, B1, &w.mem_bsoff)) || (rc = bind(k++, N1, &w.row_len)) || (rc = bind(k++, size_t(8), &w.err)) ||
-      (rc = bind(k++, N1, &w.large_list)) || (rc = bind(k++, N1, &w.is_large)))
+      (rc = bind(k++, N1, &w.large_list)))
     return rc;
   w.n_large = w.err + 1;
   w.ticket = w.err + 2;
