@@ -264,6 +264,7 @@ __device__ __forceinline__ void set_err(const Work& w, int bits) {
 // Whether an error was reported before the block came to look, as one answer for all of
 // its threads: blocks of the same launch report errors too, and a wavefront that left on
 // its own reading would leave the others without what it sets up for the block.
+// What a kernel needs next is best loaded before the call, which waits for the word.
 __device__ __forceinline__ bool block_stops(const int* err) {
   __shared__ int stop;
   if (threadIdx.x == 0) stop = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1830,12 +1831,12 @@ __global__ void __launch_bounds__(kBlock, kDescribeWavesPerSimd) k_describe(DevV
   // of them one after another on the wavefront that met them ended the kernel 10 us late
   constexpr int kList = 128;
   __shared__ int list[kList], n_list;
+  const int n_groups = n_groups_of(w);
   if (threadIdx.x == 0) n_list = 0;
   if (block_stops(w.err)) return;  // an invalid view was detected: nothing below may trust it
   const int lane = threadIdx.x % kWave;
   const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   DescribeShared& S = shared[wid];
-  const int n_groups = n_groups_of(w);
   // more row groups than the view's DoF signatures give have no room for records
   if (n_groups > w.meta_cap && blockIdx.x == 0 && threadIdx.x == 0) set_err(w, kErrView);
   const int n = min(n_groups, w.meta_cap);
@@ -2008,12 +2009,12 @@ template <bool kLibInLds, bool kACurlCurl, bool kBCurlCurl, int P>
 __global__ void __launch_bounds__(kFillBlock, kFillWavesPerSimd) k_fill_flat(Work w, LibShape L, FillOut o) {
   using VA = typename Store<P>::A;
   using VB = typename Store<P>::B;
+  const long long nnz = w.row_ptr[w.n_dofs];
   if (block_stops(w.err)) return;  // so that every wavefront is there to ask for tickets and to answer
   __shared__ FillShared shared[kFillBlock / kWave];
   __shared__ FillRounds rounds;
   // the block's copy of the Gram library (when it fits)
   __shared__ double lib_lds[kLibInLds ? kFillLibLds : 1];
-  const long long nnz = w.row_ptr[w.n_dofs];
   if (nnz > o.capacity) return;  // the host grows the buffers and runs the fill again
   const long long chunk = uniform(fill_chunk(w, nnz));
   const long long n_chunks = min((nnz + chunk - 1) / chunk, w.chunk_cap);
@@ -2489,10 +2490,10 @@ __device__ bool build_group(const DevView& v, const Work& w, int g, GroupShared&
 }
 
 __global__ void __launch_bounds__(kBlock) k_count_large(DevView v, Work w) {
-  if (block_stops(w.err)) return;  // an invalid view was detected: nothing below may trust it
-  extern __shared__ unsigned char smem[];
-  GroupShared& S = *reinterpret_cast<GroupShared*>(smem);
   const int n_large = *w.n_large;
+  if (block_stops(w.err)) return;  // an invalid view was detected: nothing below may trust it
+  extern __shared__ __align__(16) unsigned char smem[];
+  GroupShared& S = *reinterpret_cast<GroupShared*>(smem);
   for (int i = blockIdx.x; i < n_large; i += gridDim.x) {
     const int g = w.large_list[i];
     const int r0 = w.g_start[g], r1 = w.g_start[g + 1];
@@ -2517,13 +2518,13 @@ __global__ void __launch_bounds__(kBlock) k_count_large(DevView v, Work w) {
 // spec list before it is used; a violation sets kErrView and the entry is
 // skipped.
 __global__ void __launch_bounds__(kBlock) k_fill_large(DevView v, Work w, LibShape L, FillOut o) {
+  const int n_large = *w.n_large;
+  const long long nnz = w.row_ptr[w.n_dofs];
   if (block_stops(w.err)) return;  // an invalid view was detected: nothing below may trust it
-  // the host grows the buffers and runs the assembly again (as k_fill_flat)
-  if (w.row_ptr[w.n_dofs] > o.capacity) return;
-  extern __shared__ unsigned char smem[];
+  if (nnz > o.capacity) return;    // the host grows the buffers and runs the assembly again (as k_fill_flat)
+  extern __shared__ __align__(16) unsigned char smem[];
   GroupShared& S = *reinterpret_cast<GroupShared*>(smem);
   const int64_t* __restrict__ row_ptr = w.row_ptr;
-  const int n_large = *w.n_large;
   for (int i = blockIdx.x; i < n_large; i += gridDim.x) {
     const int g = w.large_list[i];
     const int r0 = w.g_start[g], r1 = w.g_start[g + 1];
