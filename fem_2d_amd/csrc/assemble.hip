@@ -947,20 +947,17 @@ __device__ __forceinline__ int src_slot(int g, int n_src) {
 }
 
 // CSR layout by row groups. Item g is the length of group g's segment: row q
-// of a streaming-fill group holds T - q entries, so the segment is
-// nrows T - nrows (nrows - 1) / 2 long; a block-path group sums the row
-// lengths its count kernel wrote. The exclusive sum is the segment's first
-// entry.
+// holds T - q entries, so the segment is nrows T - nrows (nrows - 1) / 2 long (the
+// count kernel wrote a block-path group's T, its first row's length). The
+// exclusive sum is the segment's first entry.
 struct GroupScan {
   static constexpr int kRounds = 1;
   Work w;
   __device__ long long load(long long g) const {
     if (*w.err || g >= n_groups_of(w)) return 0;
     const int4 hdr = w.meta_hdr[g];
-    if (hdr.x > 0) return (long long)hdr.y * hdr.x - (long long)hdr.y * (hdr.y - 1) / 2;
-    long long len = 0;
-    for (int r = w.g_start[g]; r < w.g_start[g + 1]; ++r) len += w.row_len[r];
-    return len;
+    const long long T = hdr.x > 0 ? hdr.x : w.row_len[w.g_start[g]];
+    return hdr.y * T - (long long)hdr.y * (hdr.y - 1) / 2;
   }
 };
 
@@ -1165,8 +1162,9 @@ __global__ void __launch_bounds__(kBlock) k_scan_apply(long long n, Op op, const
 // segment (a group with many of them gets its whole wavefront). The item past the
 // last group carries nnz and writes the call's status block (nnz, error bits,
 // block-path groups, row groups). Without tile_sum (few groups) every block sums the
-// groups before its own, and `parts` blocks share a tile's chunks (94 groups of 3 700
-// entries: 13.8 us with one block, 5.2 with eight).
+// groups before its own. `parts` blocks share a tile's chunks: the groups' segments may
+// be long (94 groups of 3 700 entries 13.8 us with one block a tile, 5.2 with eight;
+// 2 856 groups of 4 850 entries 20.0 and 5.5).
 __global__ void __launch_bounds__(kBlock) k_layout(Work w, long long n_items, const long long* tile_sum,
                                                    int parts) {
   __shared__ long long s_wave[kWavesPerBlock], s_pre[kWavesPerBlock], s_all[kWavesPerBlock];
@@ -1230,9 +1228,11 @@ __global__ void __launch_bounds__(kBlock) k_layout(Work w, long long n_items, co
     if (!real || (part > 0 && hdr.x <= 0)) c1 = c;
     if (real && hdr.x <= 0 && part == 0) {  // a block-path group
       long long at = start;
-      for (int r = w.g_start[g]; r < w.g_start[g + 1]; ++r) {
+      const int r0 = w.g_start[g];
+      const long long T = w.row_len[r0];
+      for (int r = r0; r < r0 + hdr.y; ++r) {
         w.row_ptr[r] = at;
-        at += w.row_len[r];
+        at += T - (r - r0);
         for (; c < c1 && c * C < at; ++c) w.chunk_first[c] = r;
       }
     }
@@ -3306,7 +3306,7 @@ int launch_prep(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, bool fine_eve
   // pass sums the tiles itself (a launch less)
   constexpr long long kLayoutTiles = 8;
   const bool two_pass = a.tiles_grp > kLayoutTiles;
-  const int parts = two_pass ? 1 : 8;
+  const int parts = int(std::max(1LL, std::min(8LL, 128 / a.tiles_grp)));
   if (two_pass) k_scan_reduce<<<scan_grid(a.tiles_grp), kBlock, 0, st>>>(a.n_grp_items, GroupScan{w}, a.ts_grp);
   k_layout<<<scan_grid(a.tiles_grp) * unsigned(parts), kBlock, 0, st>>>(w, a.n_grp_items,
                                                                         two_pass ? a.ts_grp : nullptr, parts);
