@@ -911,27 +911,42 @@ __device__ __forceinline__ void segment_row(int p, int T, int nrows, float bq, i
   q += up ? 1 : 0;
 }
 
-// CSR entries per chunk of the streaming fill: a multiple of kWave such that nnz
-// entries make whole rounds of one chunk a wavefront, in as few rounds as chunks of
-// max_chunk entries allow. A chunk costs a chain of dependent loads before its
-// first entry, so few large ones are faster (25.7 M entries, FP64: 256 entries
-// 113 us, 384 101, 512 100, 768 111; FP32: 512 87, 640 82, 768 84, 1024 85) until a
-// round leaves wavefronts idle (5.2 M entries: 320 51 us, 512 55, 1024 73). The
-// table of first rows (cap chunks) may demand larger ones.
-__host__ __device__ __forceinline__ int fill_chunk_of(long long nnz, long long cap, int waves, int max_chunk) {
-  const long long round = (long long)waves * max_chunk;
-  const long long rounds = nnz > round ? (nnz + round - 1) / round : 1;
-  long long c = (nnz + waves * rounds - 1) / (waves * rounds);
+// CSR entries per chunk of the streaming fill, a multiple of kWave. A chunk costs a chain
+// of dependent loads before its first entry, so few large ones are faster (25.7 M
+// entries, FP64: 256 entries 111 us, 384 99, 512 100, 768 108; FP32: 512 84, 640 80,
+// 768 82), as long as the last ones do not keep the rest waiting: about five a wavefront
+// (6.0 M entries of 31 a row: 320 41 us, 512 45; FP32 320 40, 768 45), and ten from 640
+// entries on (FP32, 22.4 M: 640 99 us, 768 112; 37.6 M: 640 137, 768 128). Not below 256
+// entries (3.4 M of 31 a row: 192 33 us, 256 31, 448 35) or about 12 rows (1.3 M of 12 a
+// row: 128 30 us, 256 45; 0.9 M of 5 a row: 64 54, 256 80). One chunk each does what takes
+// a wavefront up to 12 rows (1.6 M of 57 a row: 448 18 us, 256 21; 0.5 M of 12 a row: 192
+// 27, 128 28) or would make less than one and a half. The table of first rows (cap chunks)
+// may demand larger ones.
+__host__ __device__ __forceinline__ int fill_chunk_of(long long nnz, long long n_dofs, long long cap, int waves,
+                                                      int max_chunk) {
+  constexpr long long kOnce = 640, kRowsOnce = 12, kLeast = 256;
+  const long long each = (nnz + waves - 1) / waves;
+  long long c = each;
+  if (each > kOnce || n_dofs > kRowsOnce * waves) {
+    const long long rows = kRowsOnce * nnz / n_dofs, few = rows < kLeast ? rows : kLeast;
+    c = each / 5 > few ? each / 5 : few;
+    if (c > kOnce) c = each / 10 > kOnce ? each / 10 : kOnce;
+    if (c > max_chunk) c = max_chunk;
+    c = 3 * c > 2 * each ? each : (c + kWave / 2) / kWave * kWave;
+  }
   const long long least = (nnz + cap - 1) / cap;
   if (c < least) c = least;
   if (c < 1) c = 1;
   return int((c + kWave - 1) / kWave * kWave);
 }
 // entries of the table of first rows for the chunks that fill_chunk_of makes of up to
-// `capacity` entries
-long long fill_chunk_cap(long long capacity, int waves, int max_chunk) { return capacity / max_chunk + waves + 1; }
+// `capacity` entries: of max_chunk entries, or fewer than eight a wavefront, or of eight
+// rows and more
+long long fill_chunk_cap(long long capacity, long long n_dofs, int waves, int max_chunk) {
+  return capacity / max_chunk + 8LL * waves + n_dofs / 8 + 1;
+}
 __device__ __forceinline__ int fill_chunk(const Work& w, long long nnz) {
-  return w.chunk ? w.chunk : fill_chunk_of(nnz, w.chunk_cap, w.fill_waves, w.chunk_max);
+  return w.chunk ? w.chunk : fill_chunk_of(nnz, w.n_dofs, w.chunk_cap, w.fill_waves, w.chunk_max);
 }
 
 // First column record and first source record of row group g inside its slots of
@@ -2020,33 +2035,13 @@ __global__ void __launch_bounds__(kFillBlock, kFillWavesPerSimd) k_fill_flat(Wor
   const long long n_chunks = min((nnz + chunk - 1) / chunk, w.chunk_cap);
   constexpr int kWaves = kFillBlock / kWave;
   if (blockIdx.x * (long long)kWaves >= n_chunks) return;  // no chunk for this block
-  if (kLibInLds) {
-    const int n_lib = (L.nr + L.nr_v) * L.range_stride;
-    for (int i = threadIdx.x; i < n_lib; i += blockDim.x) lib_lds[i] = w.lib[i];
-  }
+  // the first ticket (none is needed where one round does it) and the first chunk's rows
+  // load while the library is copied
+  int asked0 = 0;
+  if (threadIdx.x == 0 && gridDim.x * (long long)kWaves < n_chunks) asked0 = atomicAdd(w.ticket, 1);
   const int lane = threadIdx.x % kWave;
   FillShared& S = shared[threadIdx.x / kWave];
   const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
-  auto answer = [&](int k, int t) {  // one lane
-    __hip_atomic_store(&rounds.ring[k % kRing], ((unsigned long long)unsigned(k + 1) << 32) | (gridDim.x + unsigned(t)),
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  };
-  for (int i = threadIdx.x; i < kRing; i += blockDim.x) rounds.ring[i] = i == 0 ? (1ull << 32) | blockIdx.x : 0ull;
-  if (threadIdx.x == 0) rounds.claimed = 2;
-  __syncthreads();
-  if (threadIdx.x == 0) answer(1, atomicAdd(w.ticket, 1));
-  // this wavefront's chunk of the block's round k (past the last chunk at the end)
-  auto take = [&](int k) -> long long {
-    unsigned long long v;
-    while (true) {
-      v = __hip_atomic_load(&rounds.ring[k % kRing], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      if (__builtin_amdgcn_readfirstlane(int(v >> 32)) == k + 1) break;
-      __builtin_amdgcn_s_sleep(1);
-    }
-    return (long long)unsigned(__builtin_amdgcn_readfirstlane(int(v))) * kWaves + wid;
-  };
-  const double* __restrict__ lib = kLibInLds ? lib_lds : w.lib;
-  const int tab = L.tab;
   // lanes l and l + kBatchRows work on row l of a batch: the first on its spec on
   // the group's first Elem, the other on the one on its second
   const int row = lane % kBatchRows, k = lane / kBatchRows;
@@ -2067,10 +2062,34 @@ __global__ void __launch_bounds__(kFillBlock, kFillWavesPerSimd) k_fill_flat(Wor
     hdr_ahead = w.meta_hdr[g_ahead - 1];
     seg_ahead = w.seg_start[g_ahead - 1];
   };
-  long long ch_next = take(0);
+  long long ch_next = blockIdx.x * (long long)kWaves + wid;
   int r = ch_next < n_chunks ? ld_const(w.chunk_first, ch_next) : 0;  // the batch's first row, which holds entry `pos`
   load_rows(r);
+  if (kLibInLds) {
+    const int n_lib = (L.nr + L.nr_v) * L.range_stride;
+    for (int i = threadIdx.x; i < n_lib; i += blockDim.x) lib_lds[i] = w.lib[i];
+  }
   load_groups();
+  auto answer = [&](int k, int t) {  // one lane
+    __hip_atomic_store(&rounds.ring[k % kRing], ((unsigned long long)unsigned(k + 1) << 32) | (gridDim.x + unsigned(t)),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  for (int i = threadIdx.x; i < kRing; i += blockDim.x) rounds.ring[i] = i == 0 ? (1ull << 32) | blockIdx.x : 0ull;
+  if (threadIdx.x == 0) rounds.claimed = 2;
+  __syncthreads();
+  if (threadIdx.x == 0) answer(1, asked0);
+  // this wavefront's chunk of the block's round k (past the last chunk at the end)
+  auto take = [&](int k) -> long long {
+    unsigned long long v;
+    while (true) {
+      v = __hip_atomic_load(&rounds.ring[k % kRing], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (__builtin_amdgcn_readfirstlane(int(v >> 32)) == k + 1) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    return (long long)unsigned(__builtin_amdgcn_readfirstlane(int(v))) * kWaves + wid;
+  };
+  const double* __restrict__ lib = kLibInLds ? lib_lds : w.lib;
+  const int tab = L.tab;
   for (int round = 0;; ++round) {
     const long long ch = ch_next;
     if (ch - wid >= n_chunks) break;  // the block's last round (every wavefront's)
@@ -3787,7 +3806,7 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
       return rc;
     const FillOut o = make_fill_out(precision, ai, bi, ctx->out_capacity, static_cast<int*>(ctx->out_col.p),
                                     ctx->out_a.p, ctx->out_b.p, static_cast<unsigned*>(ctx->out_r.p));
-    w.chunk_cap = w.chunk ? o.capacity / w.chunk + 1 : fill_chunk_cap(o.capacity, w.fill_waves, w.chunk_max);
+    w.chunk_cap = w.chunk ? o.capacity / w.chunk + 1 : fill_chunk_cap(o.capacity, nd, w.fill_waves, w.chunk_max);
     if ((rc = slot(ctx, kChunkSlot, size_t(w.chunk_cap), &w.chunk_first))) return rc;
     const bool fill = o.capacity > 0;
     const bool tail = fill && run_large;  // part (c) has work
@@ -3861,7 +3880,7 @@ int fem2d_assemble_device(fem2d_ctx* ctx, const fem2d_device_domain* dd, int bas
   }
   dd->large_state = n_large > 0 ? 1 : 0;
   if (ctx->use_graphs) ctx->graph_rule.learned(n_large > 0);
-  ctx->timing.fill_chunk = w.chunk ? w.chunk : fill_chunk_of(nnz, w.chunk_cap, w.fill_waves, w.chunk_max);
+  ctx->timing.fill_chunk = w.chunk ? w.chunk : fill_chunk_of(nnz, w.n_dofs, w.chunk_cap, w.fill_waves, w.chunk_max);
   ctx->timing.fill_lib_lds = fill_place(a.lib_n);
 
   out->n = nd;
@@ -3927,7 +3946,7 @@ int fem2d_assemble_device_noalloc(fem2d_ctx* ctx, const fem2d_device_domain* dd,
   const size_t at = (used + 255) & ~size_t(255);
   const long long left = at < kScratchBytes ? (long long)((kScratchBytes - at) / sizeof(int)) : 0;
   w.chunk_cap = w.chunk ? capacity / w.chunk + 1
-                        : std::max<long long>(std::min<long long>(fill_chunk_cap(capacity, w.fill_waves, w.chunk_max), left),
+                        : std::max<long long>(std::min<long long>(fill_chunk_cap(capacity, w.n_dofs, w.fill_waves, w.chunk_max), left),
                                    capacity / kMaxChunk + 1);
   w.chunk_first = static_cast<int*>(carve(size_t(w.chunk_cap) * sizeof(int)));
   if (used > kScratchBytes) {
