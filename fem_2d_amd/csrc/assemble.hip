@@ -1973,7 +1973,8 @@ struct __attribute__((aligned(16))) SourceTail {
 // by ticket, and 315-330 us with the same chunks dealt out in advance, whether to
 // resident blocks or block by block. A ticket costs 12 ns (one address, beyond the XCDs'
 // L2 caches), so rounds of less than about 16 x 256 entries are bound by it.
-// A block's first round is its own number. The first wavefront of a block to begin
+// A block's first round is its own number; it asks for the second one's ticket as it
+// starts, unless one round of all blocks does it. The first wavefront of a block to begin
 // its round k asks for round k + 2 once it has seen the ticket of round k + 1 (so
 // a block's tickets ascend, and the first one past the end is its last), and
 // passes the answer on when its chunk is written. kRing tickets are kept, and a barrier every
@@ -3352,8 +3353,9 @@ int launch_large_fill(fem2d_ctx* ctx, hipStream_t st, const Assembly& a, const F
   return FEM2D_OK;
 }
 
-// resident blocks of the streaming fill of one stored precision (the fill
-// assigns its chunks statically: exactly these are launched)
+// resident blocks of the streaming fill of one stored precision: exactly these are
+// launched (they take rounds of chunks until none is left), and the chunk size follows
+// from their wavefronts
 template <int P>
 int fill_grids(fem2d_ctx* ctx) {
   int per_cu = 0;

@@ -490,7 +490,6 @@ __global__ void k_shifted(long long n, const double* __restrict__ ax, const doub
     out[i] = ax[i] - sigma * bx[i];
 }
 
-// dst[p] = src[perm[p]] (to level order) or dst[perm[p]] = src[p] (back)
 // The modified Gram-Schmidt step i of GMRES on the new direction w: w = ax - sigma bx
 // (i = 0) or w -= (w . vp) vp, with the dot product's parts from step i - 1, and
 // per block the parts of w . vn (w . w when vn is null) for the next one. The
@@ -532,6 +531,7 @@ __global__ void __launch_bounds__(kBlock) k_mgs_next(long long n, const double* 
   for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n; k += stride) v[k] = w[k] * inv;
 }
 
+// dst[p] = src[perm[p]] (to level order) or dst[perm[p]] = src[p] (back)
 __global__ void k_permute(long long n, const int* __restrict__ perm, const double* __restrict__ src,
                           double* __restrict__ dst, int back) {
   const long long stride = (long long)gridDim.x * blockDim.x;

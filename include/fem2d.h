@@ -152,7 +152,7 @@ int fem2d_ctx_synchronize(fem2d_ctx* ctx);
 /* Whether assemblies on this context are recorded as a HIP graph, the second time
  * in a row that one Domain comes with the same options and buffers, and replayed
  * (default 1) or launched kernel by kernel (0). Results are the same;
- * graphs remove the per-kernel launch gaps of the ~20-kernel pipeline. */
+ * graphs remove the launch gaps between an assembly's seven to ten kernels. */
 int fem2d_ctx_set_graphs(fem2d_ctx* ctx, int enable);
 /* Accepted for callers of earlier versions, which timed the entry fill's shapes on a
  * Domain's first assembly: its chunk size and library placement now follow from
@@ -373,18 +373,18 @@ int fem2d_xy_fields(fem2d_ctx* ctx, const fem2d_domain_view* domain, int basis, 
                     const double* solution, int64_t n_solution, double* out_x, double* out_y);
 
 /* Per-stage device time of the last assembly on this context, measured with
- * HIP events recorded on the context's stream (milliseconds). An assembly that
- * replays its recorded HIP graph (the default, fem2d_ctx_set_graphs) is timed
- * end to end only: total_ms; the stage and kernel times are those of
- * kernel-by-kernel assemblies and read 0 otherwise. */
+ * HIP events recorded on the context's stream (milliseconds). With graphs (the
+ * default, fem2d_ctx_set_graphs) an assembly, replayed or launched, is timed
+ * end to end only: total_ms; the stage and kernel times are those of assemblies
+ * without graphs and read 0 otherwise. */
 typedef struct fem2d_timing {
   double total_ms;    /* first to last event of the assembly */
   double prep_ms;     /* elem geometry, DoF signatures, row groups, Gram tables */
   double symbolic_ms; /* per-group column sets and row lengths, row_ptr scan */
   double fill_ms;     /* column, A and B values of every stored entry */
   int64_t n_groups;   /* row groups (runs of DoFs whose basis specs share their Elems) */
-  double count_kernel_ms; /* the wave-per-group row-length kernel alone */
-  double fill_kernel_ms;  /* the wave-per-group entry-writing kernel alone */
+  double count_kernel_ms; /* the kernel that describes the row groups, alone */
+  double fill_kernel_ms;  /* the streaming entry-writing kernel alone (large row groups' not included) */
   int64_t nnz;
   int64_t n_large;    /* row groups assembled one block per group (large column sets) */
   int64_t fill_chunk; /* CSR entries per work item of the entry fill */
