@@ -81,8 +81,8 @@ def solve_gep_sparse(gep: Union[GEP, N.GepDevice], target_eigenvalue: float,
 
 
 # the dense solve is used up to this many DoFs by slepc_solve_gep, the sparse one beyond (at 4496
-# DoFs the dense solve takes 106-154 ms, its LU panels and substitutions latency-bound, the sparse
-# one 36 ms; at 1096 both take ~15 ms)
+# DoFs the dense solve takes 95-160 ms, its LU panels and substitutions latency-bound, the sparse
+# one 28 ms; at 1096 both take ~10 ms)
 SLEPC_DENSE_LIMIT = 2048
 
 
