@@ -270,3 +270,19 @@ def test_first_row_table_short_of_scratch():
         check_same(ctx, dom, (8, 8), F.HierPoly, precision).free()
     nothing.free()
     ctx.close()
+
+
+# the rule's branches: one chunk a wavefront, 12 rows, 256 entries, five chunks a wavefront
+@pytest.mark.parametrize("nx,order,chunk", [(32, 4, 384), (96, 2, 128), (48, 4, 256), (64, 4, 320)])
+def test_chunk_rule(ctx, nx, order, chunk):
+    """The automatic chunk size (of the 4 096 wavefronts of 256 CUs) and a forced one give the same bits."""
+    print(f"[shapes] chunk rule {nx}x{nx // 2} order={order}", flush=True)
+    dd = F.DeviceDomain(F.Domain.from_mesh(W.waveguide_64x32_mesh(nx, nx // 2, order=order, levels=2)), ctx)
+    got = dd.download(dd.assemble((8, 8), F.HierPoly))
+    assert ctx.last_timing()["fill_chunk"] == chunk
+    ctx.set_fill_chunk(512)
+    try:
+        ref = dd.download(dd.assemble((8, 8), F.HierPoly))
+    finally:
+        ctx.set_fill_chunk(0)
+    _same_bits(got, ref)
